@@ -215,6 +215,15 @@ int ygg_float_load(const ygg_float_desc *desc, int precision, int device, ygg_fm
 int ygg_float_run(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, void *d_state, void *d_logits,
                   int32_t *d_leaves, double *d_stats, void *stream);
 
+/* ygg_float_run of a call whose tokens are all known, layer by layer over the whole call instead of token by token (only
+   the recurrence inside a layer is sequential): the same arguments and results, its sums in another order, and device
+   scratch of scratch_bytes, 256-byte aligned, that no other call uses until this one has run. ygg_float_scratch gives
+   the bytes a call of B streams and T tokens wants (at most 1 GiB, or 64 rows' worth; with less the call goes in more
+   and shorter chunks), or 0 where ygg_float_run_scratch takes ygg_float_run's way and needs none. */
+int64_t ygg_float_scratch(const ygg_fmodel *m, int B, int T);
+int ygg_float_run_scratch(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, void *d_state, void *d_logits,
+                          int32_t *d_leaves, double *d_stats, void *d_scratch, int64_t scratch_bytes, void *stream);
+
 /* Wait for `stream`, then return and clear the float model's error word (bit 0: a token outside [0, vocab)). */
 int ygg_float_take_errors(const ygg_fmodel *m, void *stream, uint32_t *errors);
 

@@ -16,7 +16,8 @@ LIB_PATH = Path(__file__).resolve().parent / "libygg_hip.so"
 # every entry point of include/ygg_hip.h
 SYMBOLS = ("ygg_load", "ygg_load_blob", "ygg_model_info", "ygg_free", "ygg_step", "ygg_run", "ygg_run_grouped",
            "ygg_run_grouped_noalloc", "ygg_softmax", "ygg_score",
-           "ygg_generate", "ygg_take_errors", "ygg_float_load", "ygg_float_run", "ygg_float_take_errors",
+           "ygg_generate", "ygg_take_errors", "ygg_float_load", "ygg_float_run", "ygg_float_scratch",
+           "ygg_float_run_scratch", "ygg_float_take_errors",
            "ygg_float_free", "ygg_kernel_name", "ygg_spec_stats", "ygg_last_error", "ygg_version")
 
 ERRORS = {1: "io", 2: "format", 3: "limits", 4: "nomem", 5: "arg", 6: "token", 7: "device"}
@@ -83,6 +84,9 @@ def lib() -> ctypes.CDLL:
     L.ygg_spec_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_uint64), i32]
     L.ygg_float_load.argtypes = [ctypes.POINTER(FloatDesc), i32, i32, ctypes.POINTER(vp)]
     L.ygg_float_run.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp]
+    L.ygg_float_scratch.argtypes = [vp, i32, i32]
+    L.ygg_float_scratch.restype = ctypes.c_int64
+    L.ygg_float_run_scratch.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp, ctypes.c_int64, vp]
     L.ygg_float_take_errors.argtypes = [vp, vp, ctypes.POINTER(ctypes.c_uint32)]
     L.ygg_float_free.argtypes = [vp]
     L.ygg_float_free.restype = None

@@ -25,38 +25,11 @@
 #include <string>
 #include <vector>
 
-#include "../../include/ygg_hip.h"
-#include "ygg_layout.h"
+#include "ygg_float.h"
 
-namespace ygg {
-int set_error(int code, const char *msg);
-}
+using namespace ygg::flt;
 
 namespace {
-
-constexpr int kMaxN = 256, kMaxR = 64, kMaxR2 = 64, kMaxClasses = 256, kMaxF = 256, kMaxB = 16;
-constexpr double kRmsEps = 1e-6;   // yggdrasil/config.py:8
-
-// Device layouts: the arrays a thread reads a row of at each step of a dot are stored transposed from the checkpoint's,
-// so that the lanes of a wavefront read consecutive addresses at every step.
-template <typename T> struct FloatLayerDev {
-    const T *table;          // token layer [V][n] (T_x[x]); routed [E][V][n]
-    const T *A;              // [E][n/b][b (column j)][b (row i)] (each block transposed) or null
-    const T *P;              // [E][R][n]
-    const T *Q;              // [R][classes] (transposed)
-    const T *emb;            // routed: [V][F]
-    const T *W;              // routed: [nodes][F + n] (router_state) or [nodes][F]
-    const T *bias;           // routed: [nodes]
-    const T *Vd;             // [n][R2] (transposed) or null
-    const T *Up;             // [E][R2][n] (each expert's matrix transposed) or null
-};
-
-template <typename T> struct FloatDevModel {
-    int L, n, b, V, classes, D, R, R2, F, router_state;
-    const T *output_bias;    // [classes]
-    uint32_t *err;
-    FloatLayerDev<T> layers[YGG_MAX_LAYERS];
-};
 
 constexpr int kFThreads = 256;
 
@@ -259,12 +232,23 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                 const bool up = l > 0 && y.Up != nullptr, ta = y.A != nullptr;
                 const int g = i / b, ii = i % b;
                 const T *u = up ? y.Up + (size_t)r * R2 * n + i : nullptr;                    // column i
-                const T *acol = ta ? y.A + ((size_t)r * (n / b) + g) * b * b + ii : nullptr;  // row ii of block g
+                const T *ablk = ta ? y.A + ((size_t)r * (n / b) + g) * b * b : nullptr;       // block g
                 T uw[MR2], aw[MB];
 #pragma unroll
                 for (int k = 0; k < MR2; k++) uw[k] = (up && k < R2) ? u[(size_t)k * n] : T(0);
+                if (ta && b == 16) {     // (whole 16-byte chunks of row ii)
+                    constexpr int VE = 16 / (int)sizeof(T);
+                    struct alignas(16) Chunk { T v[VE]; };
 #pragma unroll
-                for (int j = 0; j < MB; j++) aw[j] = (ta && j < b) ? acol[j * b] : T(0);
+                    for (int j = 0; j < MB / VE; j++) {
+                        const Chunk w = *(const Chunk *)(ablk + a_index<T>(16, ii, j * VE));
+#pragma unroll
+                        for (int e = 0; e < VE; e++) aw[j * VE + e] = w.v[e];
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < MB; j++) aw[j] = (ta && j < b) ? ablk[a_index<T>(b, ii, j)] : T(0);
+                }
                 T h = trow[i];
                 if constexpr (PF) load_p();
                 if (up) {
@@ -346,7 +330,9 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
     }
 }
 
-int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
+}  // namespace
+
+namespace ygg::flt {
 int fail(int code, const char *fmt, ...) {
     char buf[512];
     va_list ap;
@@ -355,34 +341,7 @@ int fail(int code, const char *fmt, ...) {
     va_end(ap);
     return ygg::set_error(code, buf);
 }
-
-#define HIP_TRY(expr)                                                                                  \
-    do {                                                                                               \
-        hipError_t e_ = (expr);                                                                        \
-        if (e_ != hipSuccess) return fail(YGG_ERR_DEVICE, "%s: %s", #expr, hipGetErrorString(e_));     \
-    } while (0)
-
-struct DeviceGuard {
-    int prev = -1;
-    hipError_t set(int dev) {
-        hipError_t e = hipGetDevice(&prev);
-        if (e != hipSuccess) { prev = -1; return e; }
-        return hipSetDevice(dev);
-    }
-    ~DeviceGuard() {
-        if (prev >= 0) (void)hipSetDevice(prev);
-    }
-};
-
-}  // namespace
-
-struct ygg_fmodel {
-    int device = 0, precision = 32;
-    void *arena = nullptr;
-    size_t arena_bytes = 0;
-    FloatDevModel<float> m32{};
-    FloatDevModel<double> m64{};
-};
+}  // namespace ygg::flt
 
 namespace {
 
@@ -390,13 +349,14 @@ template <typename T> int upload(const ygg_float_desc *d, int device, ygg_fmodel
     const int L = d->n_layers, n = d->d_state, b = d->block_size, V = d->vocab, C = d->classes, D = d->router_depth,
               R = d->readout_rank, R2 = d->layer_input_rank, F = d->router_token_dim;
     const int64_t E = (int64_t)1 << D, nodes = E - 1, width = F + (d->router_state ? n : 0);
-    // a part is `outer` matrices of rows x cols, stored as given (rows = 0) or each transposed
-    struct Part { const double *src; int64_t count; size_t off; int64_t outer, rows, cols; };
+    // a part is `outer` matrices of rows x cols, stored as given (rows = 0), each transposed, or (block) as a_index
+    // places a transition block
+    struct Part { const double *src; int64_t count; size_t off; int64_t outer, rows, cols; bool block; };
     std::vector<Part> parts;
     size_t total = 256;   // the error word first
-    auto add = [&](const double *src, int64_t count, int64_t rows = 0, int64_t cols = 0) -> int {
+    auto add = [&](const double *src, int64_t count, int64_t rows = 0, int64_t cols = 0, bool block = false) -> int {
         if (!src || count <= 0) return -1;
-        parts.push_back({src, count, total, rows ? count / (rows * cols) : 0, rows, cols});
+        parts.push_back({src, count, total, rows ? count / (rows * cols) : 0, rows, cols, block});
         total += ((size_t)count * sizeof(T) + 255) / 256 * 256;
         return (int)parts.size() - 1;
     };
@@ -404,14 +364,19 @@ template <typename T> int upload(const ygg_float_desc *d, int device, ygg_fmodel
     if (ob < 0) return fail(YGG_ERR_ARG, "float model: output_bias is NULL");
     struct Idx { int table, A, P, Q, emb, W, bias, Vd, Up; };
     std::vector<Idx> idx(L);
+    // the layers' transposed unembeddings one after the other: [L R][classes]
+    for (int l = 0; l < L; l++) {
+        idx[l].Q = add(d->layers[l].unembed, (int64_t)C * R, C, R);
+        if (idx[l].Q >= 0) total = parts.back().off + (size_t)C * R * sizeof(T);
+    }
+    total = (total + 255) / 256 * 256;
     for (int l = 0; l < L; l++) {
         const ygg_float_layer &y = d->layers[l];
         const int64_t El = l == 0 ? V : E;
         Idx &k = idx[l];
         k.table = add(y.table, l == 0 ? (int64_t)V * n : El * V * n);
-        k.A = add(y.transition, El * n * b, b, b);
+        k.A = add(y.transition, El * n * b, b, b, true);
         k.P = add(y.readout, El * R * n);
-        k.Q = add(y.unembed, (int64_t)C * R, C, R);
         k.emb = l ? add(y.router_embed, (int64_t)V * F) : -1;
         k.W = l ? add(y.router_weight, nodes * width) : -1;
         k.bias = l ? add(y.router_bias, nodes) : -1;
@@ -440,7 +405,9 @@ template <typename T> int upload(const ygg_float_desc *d, int device, ygg_fmodel
         const int64_t mat = p.rows * p.cols;
         for (int64_t o = 0; o < p.outer; o++)
             for (int64_t r = 0; r < p.rows; r++)
-                for (int64_t c = 0; c < p.cols; c++) dst[o * mat + c * p.rows + r] = (T)p.src[o * mat + r * p.cols + c];
+                for (int64_t c = 0; c < p.cols; c++)
+                    dst[o * mat + (p.block ? a_index<T>((int)p.rows, (int)r, (int)c) : c * p.rows + r)] =
+                        (T)p.src[o * mat + r * p.cols + c];
     }
     DeviceGuard g;
     HIP_TRY(g.set(device));

@@ -1,0 +1,838 @@
+// The float step over many known tokens, layer by layer (ygg_float_run_scratch). The step of ygg_float.hip walks a
+// stream token by token through every layer, so a token waits for all layers of the one before it. When the tokens are
+// known only one term of the step is a recurrence, h(t) = u(t) + A_r(t) h(t - 1) inside each block of 16 coordinates;
+// the route, the layer input, the expert's own input u = T_r[x] + U'_r (V' rms(h_below)) and the readout of a token need
+// nothing of the token before it in the same layer. So each layer runs over all rows (stream, token) of a chunk:
+//   fl_route    leaf and layer input of every row; 16 rows per workgroup
+//   fl_rank,    counting sort of the rows by leaf, and its tiles of at most 32 rows of one expert
+//   fl_scatter
+//   fl_input    u: per tile the product of its rows' layer inputs and the expert's U', on the f32 / f64 matrix cores,
+//               plus the table rows
+//   fl_scan     the recurrence: 16 lanes per stream and block, A_r loaded ahead by token
+// and after the last layer fl_readout (z = P_r h of every layer by the same tiles) and fl_logits (Q z, one product over
+// the layers' ranks). The rows of few tokens are not sorted (a tile is one row then).
+//
+// Measured against the token-by-token kernel (whole calls, f32 unless said): 9 streams x 100 tokens of the medium
+// trained shape 3 635 -> 224 us; scoring 256 x 128 of the large one 6 597 -> 947; f64 calibration of 500 x 200 of the
+// medium one 45.6 -> 2.15 ms. The token-by-token kernel is bound by the dependent loads and barriers of a layer (7 us
+// each), this form by its launches (17 to 26 of 4 us) at a thousand rows and by the experts' bytes at tens of thousands.
+#include <cstdlib>
+
+#include "ygg_float.h"
+
+using namespace ygg::flt;
+
+namespace {
+
+constexpr int kTile = 32;            // rows of a tile of one expert (two 16-row matrix tiles)
+constexpr int kRankRows = 2048;      // rows of one counting-sort workgroup
+constexpr int kSortLeaves = 8192;    // most experts of a layer the sort's LDS histogram holds
+
+template <typename T> struct Vec;    // the 16-byte vector of T
+template <> struct Vec<float> {
+    using type = float4;
+    static __device__ __forceinline__ float at(const float4 &v, int i) { return ((const float *)&v)[i]; }
+};
+template <> struct Vec<double> {
+    using type = double2;
+    static __device__ __forceinline__ double at(const double2 &v, int i) { return ((const double *)&v)[i]; }
+};
+template <typename T> constexpr int kVE = 16 / (int)sizeof(T);
+
+// D(16 x 16) += A(16 x 4) B(4 x 16): lane l gives A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[acc_row][l % 16]
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+template <typename T> struct Acc;
+template <> struct Acc<float> { using type = f32x4; };
+template <> struct Acc<double> { using type = f64x4; };
+__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f64x4 mma(double a, double b, f64x4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+// the row of D that component i of lane group q = l / 16 holds
+template <typename T> __device__ __forceinline__ int acc_row(int i, int q) { return sizeof(T) == 4 ? 4 * q + i : 4 * i + q; }
+
+// v moved across lanes by a DPP control (both halves of a double)
+template <int CTRL> __device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> __device__ __forceinline__ double dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// the sum over aligned groups of 16 lanes, in every lane
+template <typename T> __device__ __forceinline__ T sum16(T v) {
+    v += dpp<0xB1>(v);     // quad_perm 1 0 3 2
+    v += dpp<0x4E>(v);     // quad_perm 2 3 0 1
+    v += dpp<0x141>(v);    // row_half_mirror
+    v += dpp<0x140>(v);    // row_mirror
+    return v;
+}
+template <typename T> __device__ __forceinline__ T load_or_zero(const T *p, bool ok) { return ok ? *p : T(0); }
+template <typename T> __device__ __forceinline__ typename Vec<T>::type load_vec(const T *p, bool ok) {
+    typename Vec<T>::type v{};
+    if (ok) v = *(const typename Vec<T>::type *)p;
+    return v;
+}
+
+// One chunk of a call: Bc streams from s0, Tc of their Tn tokens from t0; row i = s Tc + t. Workspace arrays per layer
+// lie N rows apart.
+template <typename T> struct Chunk {
+    const int32_t *tokens;
+    int Tn, s0, Bc, t0, Tc, N;
+    int E, ZLW, ZW, sorted, max_tiles;
+    T *state, *logits;
+    int32_t *leaves;
+    double *stats;
+    T *h;             // [L][N][n]: u, then the states
+    T *zl;            // [L][N][ZLW]: layer inputs, zero past R2
+    T *z;             // [N][ZW]: readouts, layer l's at l R
+    int *leaf;        // [L][N], -1 past a stream's end
+    int *rank;        // [L][N] place of a row among its leaf's
+    int *order;       // [L][N] rows by leaf
+    int4 *tiles;      // [L][max_tiles]: leaf, first place in order, rows
+    int *ntiles;      // [L]
+    int *count;       // [L][E] rows per leaf
+    int *off;         // [L][E] a leaf's first place in order
+    int *done;        // [L] finished workgroups of fl_rank
+    int *stop;        // [Bc] a stream's first token outside [0, V), or Tn
+
+    __device__ __forceinline__ int len(int s) const {     // rows of stream s this chunk computes
+        const int k = stop[s] - t0;
+        return k < 0 ? 0 : (k < Tc ? k : Tc);
+    }
+    __device__ __forceinline__ size_t token_at(int row) const {
+        const int s = row / Tc;
+        return (size_t)(s0 + s) * Tn + t0 + (row - s * Tc);
+    }
+};
+
+// a tile's leaf, first place and rows, or no rows; unsorted rows are tiles of one (i the same in the whole wavefront)
+template <typename T> __device__ __forceinline__ int4 tile_at(const Chunk<T> &c, int l, int i) {
+    int4 t;
+    if (c.sorted) {
+        t = c.tiles[(size_t)l * c.max_tiles + i];
+    } else {
+        const int r = c.leaf[(size_t)l * c.N + i];
+        t = make_int4(r, i, r >= 0 ? 1 : 0, 0);
+    }
+    return make_int4(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y),
+                     __builtin_amdgcn_readfirstlane(t.z), 0);
+}
+template <typename T> __device__ __forceinline__ int row_at(const Chunk<T> &c, int l, int place) {
+    return c.sorted ? c.order[(size_t)l * c.N + place] : place;
+}
+
+// Per stream (a wavefront) its end in this chunk, and layer 0's leaves (the tokens); the sort's counters cleared. The
+// streams' ends carry over to the next chunk.
+template <typename T> __global__ __launch_bounds__(256) void fl_begin(const FloatDevModel<T> m, const Chunk<T> c) {
+    const int lane = threadIdx.x & 63, s = (blockIdx.x * 256 + threadIdx.x) >> 6;
+    if (c.sorted)
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < m.L * c.E; i += gridDim.x * 256) c.count[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < m.L) c.done[threadIdx.x] = 0;
+    if (s >= c.Bc) return;
+    int stop = c.t0 ? c.stop[s] : c.Tn;
+    const int32_t *tok = c.tokens + (size_t)(c.s0 + s) * c.Tn + c.t0;
+    for (int t = 0; t < c.Tc; t += 64) {
+        const int x = t + lane < c.Tc ? tok[t + lane] : 0;
+        const unsigned long long bad = __ballot(x < 0 || x >= m.V);
+        if (bad && c.t0 + t < stop) {
+            stop = c.t0 + t + __builtin_ctzll(bad);
+            if (lane == 0) atomicOr(m.err, 1u);
+        }
+        if (t + lane < c.Tc) {
+            const bool live = c.t0 + t + lane < stop;
+            c.leaf[(size_t)s * c.Tc + t + lane] = live ? x : -1;
+            if (live && c.leaves) c.leaves[((size_t)(c.s0 + s) * c.Tn + c.t0 + t + lane) * m.L] = x;
+        }
+    }
+    if (lane == 0) c.stop[s] = stop;
+}
+
+// The route of layer l and its layer input: 16 rows per workgroup, 16 lanes per row. The descent reads one node row per
+// level (rows of a layer stay in L2) with its input row in registers; the product V' rms(h) of the 16 rows is
+// split over the wavefronts by coordinates. EPL: router inputs per lane at most; VW: their vector width (kVE where the
+// token part is whole vectors, else 1).
+template <typename T, int EPL, int VW>
+__global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const Chunk<T> c, int l) {
+    constexpr int VE = kVE<T>, KC = 4 * VE, LD = kMaxN + VE;
+    __shared__ T f16[16][LD];                 // rms(h_below) of the rows
+    __shared__ T part[4][16][kMaxR2 + 1];
+    const FloatLayerDev<T> &y = m.layers[l];
+    const int n = m.n, F = m.F, width = F + (m.router_state ? n : 0);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rl = tid & 15, rr = tid >> 4;
+    const int row = blockIdx.x * 16 + rr;
+    const int s = row / c.Tc;
+    const bool live = row < c.N && row - s * c.Tc < c.len(s);
+    {
+        const T *h = c.h + ((size_t)(l - 1) * c.N + (live ? row : 0)) * n;
+        typename Vec<T>::type v[kMaxN / (16 * VE)];
+        T ss = T(0);
+#pragma unroll
+        for (int k = 0; k < kMaxN / (16 * VE); k++) {
+            const int e = VE * (rl + 16 * k);
+            v[k] = load_vec(h + e, live && e < n);
+#pragma unroll
+            for (int q = 0; q < VE; q++) ss = fma(Vec<T>::at(v[k], q), Vec<T>::at(v[k], q), ss);
+        }
+        const T rinv = T(1) / sqrt(sum16(ss) / T(n) + T(kRmsEps));
+#pragma unroll
+        for (int k = 0; k < kMaxN / (16 * VE); k++) {
+            const int e = VE * (rl + 16 * k);
+            if (e < n)
+#pragma unroll
+                for (int q = 0; q < VE; q++) f16[rr][e + q] = Vec<T>::at(v[k], q) * rinv;
+        }
+    }
+    __syncthreads();
+    const size_t at = live ? c.token_at(row) : 0;
+    if (live) {
+        const T *emb = y.emb + (size_t)c.tokens[at] * F;
+        T f[EPL];
+#pragma unroll
+        for (int k = 0; k < EPL / VW; k++) {
+#pragma unroll
+            for (int q = 0; q < VW; q++) {
+                const int e = VW * (rl + 16 * k) + q;
+                f[VW * k + q] = e < F ? emb[e] : (e < width ? f16[rr][e - F] : T(0));
+            }
+        }
+        int node = 0;
+        for (int d = 0; d < m.D; d++) {
+            const T *w = y.W + (size_t)node * width;
+            T p = T(0);
+            if constexpr (VW > 1) {
+                typename Vec<T>::type wv[EPL / VE];
+#pragma unroll
+                for (int k = 0; k < EPL / VE; k++) wv[k] = load_vec(w + VE * (rl + 16 * k), VE * (rl + 16 * k) < width);
+#pragma unroll
+                for (int k = 0; k < EPL / VE; k++)
+#pragma unroll
+                    for (int q = 0; q < VE; q++) p = fma(f[VE * k + q], Vec<T>::at(wv[k], q), p);
+            } else {
+                T wv[EPL];
+#pragma unroll
+                for (int k = 0; k < EPL; k++) wv[k] = load_or_zero(w + rl + 16 * k, rl + 16 * k < width);
+#pragma unroll
+                for (int k = 0; k < EPL; k++) p = fma(f[k], wv[k], p);
+            }
+            const T bias = y.bias[node];
+            node = 2 * node + 1 + (sum16(p) + bias > T(0) ? 1 : 0);
+        }
+        if (rl == 0) {
+            const int r = node - ((1 << m.D) - 1);
+            c.leaf[(size_t)l * c.N + row] = r;
+            if (c.leaves) c.leaves[at * m.L + l] = r;
+        }
+    } else if (row < c.N && rl == 0) {
+        c.leaf[(size_t)l * c.N + row] = -1;
+    }
+    if (!y.Vd) return;
+    const int R2 = m.R2, kk = lane >> 4, cl = lane & 15;
+    const bool whole = R2 % VE == 0;
+    for (int c0 = 0; c0 < R2; c0 += 16 * VE) {
+        typename Acc<T>::type acc[VE];
+#pragma unroll
+        for (int q = 0; q < VE; q++) acc[q] = typename Acc<T>::type{};
+        const int col = c0 + VE * cl;
+        for (int j = wave; j < n / KC; j += 4) {
+            const int i0 = KC * j + VE * kk;
+#pragma unroll
+            for (int u = 0; u < VE; u++) {
+                const T a = f16[cl][i0 + u];
+                const T *b = y.Vd + (size_t)(i0 + u) * R2 + col;
+                typename Vec<T>::type bv{};
+                if (whole) {
+                    bv = load_vec(b, col < R2);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < VE; q++)
+                        if (col + q < R2) ((T *)&bv)[q] = b[q];
+                }
+#pragma unroll
+                for (int q = 0; q < VE; q++) acc[q] = mma(a, Vec<T>::at(bv, q), acc[q]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < VE; q++)
+            if (col + q < kMaxR2)
+#pragma unroll
+                for (int i = 0; i < 4; i++) part[wave][acc_row<T>(i, kk)][col + q] = acc[q][i];
+    }
+    __syncthreads();
+    for (int i = tid; i < 16 * c.ZLW; i += 256) {
+        const int k = i % c.ZLW, mrow = i / c.ZLW, to = blockIdx.x * 16 + mrow;
+        if (to >= c.N) break;
+        const T z = k < R2 ? ((part[0][mrow][k] + part[1][mrow][k]) + part[2][mrow][k]) + part[3][mrow][k] : T(0);
+        c.zl[((size_t)l * c.N + to) * c.ZLW + k] = z;
+    }
+}
+
+// The counting sort's first half, for layers l0 + blockIdx.y: each workgroup counts its rows' leaves in LDS, takes the
+// leaves' places by one device-wide addition per leaf it saw (a leaf that most rows take costs one per workgroup, not
+// one per row), and the last workgroup to finish sums the counts into the leaves' first places and writes the tiles.
+template <typename T> __global__ __launch_bounds__(1024) void fl_rank(const FloatDevModel<T> m, const Chunk<T> c, int l0) {
+    extern __shared__ int hist[];
+    __shared__ int wsum[16][2], last;
+    const int l = l0 + blockIdx.y, tid = threadIdx.x, E = l == 0 ? m.V : 1 << m.D;
+    const int *leaf = c.leaf + (size_t)l * c.N;
+    int *count = c.count + (size_t)l * c.E, *off = c.off + (size_t)l * c.E;
+    for (int e = tid; e < E; e += 1024) hist[e] = 0;
+    __syncthreads();
+    constexpr int PER = kRankRows / 1024;
+    int lf[PER], at[PER];
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+        const int row = blockIdx.x * kRankRows + k * 1024 + tid;
+        lf[k] = row < c.N ? leaf[row] : -1;
+        at[k] = lf[k] >= 0 ? atomicAdd(&hist[lf[k]], 1) : 0;
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += 1024)
+        if (hist[e]) hist[e] = __hip_atomic_fetch_add(&count[e], hist[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+        if (lf[k] >= 0) c.rank[(size_t)l * c.N + blockIdx.x * kRankRows + k * 1024 + tid] = hist[lf[k]] + at[k];
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) {
+        const int before = __hip_atomic_fetch_add(&c.done[l], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        last = before == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    // exclusive sums of the counts and of the tiles, each thread a run of leaves
+    const int per = (E + 1023) / 1024, e0 = tid * per;
+    int rows = 0, tl = 0;
+    for (int e = e0; e < e0 + per && e < E; e++) {
+        const int k = __hip_atomic_load(&count[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        rows += k;
+        tl += (k + kTile - 1) / kTile;
+    }
+    const int lane = tid & 63, wave = tid >> 6;
+    int ir = rows, it = tl;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(ir, o), b = __shfl_up(it, o);
+        if (lane >= o) ir += a, it += b;
+    }
+    if (lane == 63) wsum[wave][0] = ir, wsum[wave][1] = it;
+    __syncthreads();
+    int pr = ir - rows, pt = it - tl, total = 0;
+    for (int w = 0; w < 16; w++) {
+        if (w < wave) pr += wsum[w][0], pt += wsum[w][1];
+        total += wsum[w][1];
+    }
+    int4 *tiles = c.tiles + (size_t)l * c.max_tiles;
+    for (int e = e0; e < e0 + per && e < E; e++) {
+        const int k = __hip_atomic_load(&count[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        off[e] = pr;
+        for (int q = 0; q < k; q += kTile) tiles[pt++] = make_int4(e, pr + q, k - q < kTile ? k - q : kTile, 0);
+        pr += k;
+    }
+    if (tid == 0) c.ntiles[l] = total;
+}
+
+template <typename T> __global__ __launch_bounds__(256) void fl_scatter(const Chunk<T> c, int l0) {
+    const int l = l0 + blockIdx.y;
+    const int row = blockIdx.x * 256 + threadIdx.x;
+    if (row >= c.N) return;
+    const int r = c.leaf[(size_t)l * c.N + row];
+    if (r >= 0) c.order[(size_t)l * c.N + c.off[(size_t)l * c.E + r] + c.rank[(size_t)l * c.N + row]] = row;
+}
+
+// the maximum of a non-negative v over the wavefront into *p (non-negative doubles order as their bit patterns; most
+// wavefronts find a larger one there and add nothing)
+__device__ __forceinline__ void max_into(double *p, double v, int lane) {
+    for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+    if (lane == 0 && v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax((unsigned long long *)p, (unsigned long long)__double_as_longlong(v));
+}
+
+// u = T_r[x] + U'_r zl of layer l: a wavefront per tile and 16 VE columns (each lane VE adjacent ones, so that U', the
+// table rows and u move in 16-byte pieces)
+template <typename T> __global__ __launch_bounds__(256) void fl_input(const FloatDevModel<T> m, const Chunk<T> c, int l) {
+    constexpr int VE = kVE<T>, KC = 4 * VE;
+    const FloatLayerDev<T> &y = m.layers[l];
+    const int n = m.n, R2 = m.R2, CG = (n + 16 * VE - 1) / (16 * VE);
+    const int lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
+    const int total = (c.sorted ? c.ntiles[l] : c.N) * CG;
+    double zmax = 0.0;      // (calibration) the largest layer input
+    for (int w = blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += gridDim.x * 4) {
+        const int4 tile = tile_at(c, l, w / CG);
+        const int r = tile.x, cnt = tile.z;
+        if (cnt == 0) continue;
+        const int col = (w % CG) * 16 * VE + VE * cl;
+        const bool cok = col < n, two = cnt > 16;
+        int rows[2];
+        for (int q = 0; q < 2; q++) rows[q] = row_at(c, l, tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
+        typename Acc<T>::type acc[2][VE];
+#pragma unroll
+        for (int q = 0; q < VE; q++) acc[0][q] = acc[1][q] = typename Acc<T>::type{};
+        const T *up = y.Up ? y.Up + (size_t)r * R2 * n + col : nullptr;
+        const T *z0 = c.zl + ((size_t)l * c.N + rows[0]) * c.ZLW, *z1 = c.zl + ((size_t)l * c.N + rows[1]) * c.ZLW;
+        if (up) {
+            for (int j = 0; j < c.ZLW / KC; j++) {
+                const int k0 = KC * j + VE * kk;
+                typename Vec<T>::type b[VE], a0 = load_vec(z0 + k0, true), a1 = load_vec(z1 + k0, two);
+#pragma unroll
+                for (int u = 0; u < VE; u++) b[u] = load_vec(up + (size_t)(k0 + u) * n, cok && k0 + u < R2);
+                if (c.stats)
+#pragma unroll
+                    for (int u = 0; u < VE; u++)
+                        zmax = fmax(zmax, fmax((double)fabs(Vec<T>::at(a0, u)), (double)fabs(Vec<T>::at(a1, u))));
+#pragma unroll
+                for (int u = 0; u < VE; u++)
+#pragma unroll
+                    for (int q = 0; q < VE; q++) acc[0][q] = mma(Vec<T>::at(a0, u), Vec<T>::at(b[u], q), acc[0][q]);
+                if (two)
+#pragma unroll
+                    for (int u = 0; u < VE; u++)
+#pragma unroll
+                        for (int q = 0; q < VE; q++) acc[1][q] = mma(Vec<T>::at(a1, u), Vec<T>::at(b[u], q), acc[1][q]);
+            }
+        }
+        for (int q = 0; q < 2; q++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int p = 16 * q + acc_row<T>(i, kk);
+                if (p < cnt && cok) {
+                    const int row = row_at(c, l, tile.y + p);
+                    typename Vec<T>::type t = *(const typename Vec<T>::type *)(
+                        y.table + ((size_t)r * m.V + c.tokens[c.token_at(row)]) * n + col);
+#pragma unroll
+                    for (int e = 0; e < VE; e++) ((T *)&t)[e] += q ? acc[1][e][i] : acc[0][e][i];
+                    *(typename Vec<T>::type *)(c.h + ((size_t)l * c.N + row) * n + col) = t;
+                }
+            }
+        }
+    }
+    if (c.stats) max_into(c.stats + (size_t)l * (3 + n / 16 + m.R) + 1, zmax, lane);
+}
+
+// a . h over the 16 coordinates of a block, h spread one per lane: column j's factor by a row broadcast; four partial sums
+template <typename T, int J = 0> __device__ __forceinline__ void block_dot(const T (&a)[16], T h, T (&s)[4]) {
+    if constexpr (J < 16) {
+        s[J % 4] = fma(a[J], dpp<0x150 + J>(h), s[J % 4]);
+        block_dot<T, J + 1>(a, h, s);
+    }
+}
+
+// The recurrence of layer l, h(t) = u(t) + A_r(t) h(t - 1): 16 lanes per stream and block of 16 coordinates, four
+// streams of one block per wavefront, the next PD tokens' A rows and inputs loaded ahead and the leaves PD further. The
+// loads of a token past a stream's end are those of its last one, so that every load is issued in straight-line code and
+// nothing but the token's own use waits for it. Workgroup b takes block b % (n / 16): workgroups go to the XCDs in turn,
+// so where n / 16 divides or is a multiple of 8 an XCD meets (n / 16) / 8 blocks, or one, whose share of the layer's A
+// stays in its L2. Layer 0 (L0) takes its input from the table.
+template <typename T, int PD, bool L0>
+__global__ __launch_bounds__(64) void fl_scan(const FloatDevModel<T> m, const Chunk<T> c, int l) {
+    constexpr int VE = kVE<T>, CH = 16 / VE;
+    const FloatLayerDev<T> &y = m.layers[l];
+    const int n = m.n, nb = n / 16, g = blockIdx.x % nb, lane = threadIdx.x & 63, i = lane & 15;
+    const int sw = blockIdx.x / nb * 4 + (lane >> 4), s = sw < c.Bc ? sw : c.Bc - 1;
+    const bool mine = sw < c.Bc;
+    const int len = c.len(s), last = len > 0 ? len - 1 : 0;
+    T *st = c.state + ((size_t)(c.s0 + s) * m.L + l) * n + g * 16 + i;
+    T *h = c.h + ((size_t)l * c.N + (size_t)s * c.Tc) * n + g * 16 + i;
+    const int *leaf = c.leaf + (size_t)l * c.N + (size_t)s * c.Tc;
+    // the most tokens any stream of the wavefront takes
+    int most = len;
+    for (int o = 16; o < 64; o <<= 1) {
+        const int k = __shfl_xor(most, o);
+        most = k > most ? k : most;
+    }
+    most = __builtin_amdgcn_readfirstlane(most);
+    if (most == 0) return;
+    const T *table = y.table + g * 16 + i;
+    if (!y.A) {     // no recurrence
+        T hv = *st;
+        for (int t = 0; t < len; t++) {
+            hv = L0 ? table[(size_t)leaf[t] * n] : h[(size_t)t * n];
+            if (L0 && mine) h[(size_t)t * n] = hv;
+        }
+        if (mine) *st = hv;
+        return;
+    }
+    const T *A = y.A + (size_t)g * 256 + VE * i;
+    T hv = *st;
+    typename Vec<T>::type a[PD][CH];
+    T u[PD];
+    int lf[PD];
+    auto fetch = [&](typename Vec<T>::type (&av)[CH], T &uv, int lv, int t) {
+        const int r = lv > 0 ? lv : 0;      // (a stream that stops at once has no leaf)
+        const T *ab = A + (size_t)r * nb * 256;
+#pragma unroll
+        for (int k = 0; k < CH; k++) av[k] = *(const typename Vec<T>::type *)(ab + k * 16 * VE);
+        uv = L0 ? table[(size_t)r * n] : h[(size_t)(t < last ? t : last) * n];
+    };
+#pragma unroll
+    for (int k = 0; k < PD; k++) lf[k] = leaf[k < last ? k : last];
+#pragma unroll
+    for (int k = 0; k < PD; k++) fetch(a[k], u[k], lf[k], k);
+#pragma unroll
+    for (int k = 0; k < PD; k++) lf[k] = leaf[PD + k < last ? PD + k : last];
+    for (int t0 = 0; t0 < most; t0 += PD) {
+#pragma unroll
+        for (int k = 0; k < PD; k++) {
+            const int t = t0 + k;
+            T av[16], sums[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int j = 0; j < 16; j++) av[j] = Vec<T>::at(a[k][j / VE], j % VE);
+            block_dot<T>(av, hv, sums);
+            const T hn = u[k] + ((sums[0] + sums[1]) + (sums[2] + sums[3]));
+            const bool on = t < len;
+            hv = on ? hn : hv;
+            if (on && mine) h[(size_t)t * n] = hv;
+            fetch(a[k], u[k], lf[k], t + PD);
+            lf[k] = leaf[t + 2 * PD < last ? t + 2 * PD : last];
+        }
+    }
+    if (mine) *st = hv;
+}
+
+// z = P_r h of every layer (blockIdx.y): a wavefront per tile; CT column tiles of 16 ranks, each summed in VE chains (a
+// shorter chain of additions rounds less). STATS: also the calibration maxima (cpu/export.py:127-153) of the states and
+// of the readouts; places past a tile's rows repeat its first row, which changes no maximum.
+template <typename T, int CT, bool STATS>
+__global__ __launch_bounds__(256) void fl_readout(const FloatDevModel<T> m, const Chunk<T> c) {
+    constexpr int VE = kVE<T>, KC = 4 * VE, G = kMaxN / 16;
+    const int l = blockIdx.y;
+    const FloatLayerDev<T> &y = m.layers[l];
+    const int n = m.n, R = m.R, lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
+    const int total = c.sorted ? c.ntiles[l] : c.N;
+    double hmax[STATS ? G : 1], rmax[STATS ? CT : 1];
+    for (double &v : hmax) v = 0.0;
+    for (double &v : rmax) v = 0.0;
+    for (int w = blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += gridDim.x * 4) {
+        const int4 tile = tile_at(c, l, w);
+        const int r = tile.x, cnt = tile.z;
+        if (cnt == 0) continue;
+        const bool two = cnt > 16;
+        int rows[2];
+        for (int q = 0; q < 2; q++) rows[q] = row_at(c, l, tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
+        const T *h0 = c.h + ((size_t)l * c.N + rows[0]) * n, *h1 = c.h + ((size_t)l * c.N + rows[1]) * n;
+        typename Acc<T>::type acc[2][CT][VE];
+#pragma unroll
+        for (int q = 0; q < CT; q++)
+#pragma unroll
+            for (int u = 0; u < VE; u++) acc[0][q][u] = acc[1][q][u] = typename Acc<T>::type{};
+        auto step = [&](int j) {
+            const int i0 = KC * j + VE * kk;
+            const typename Vec<T>::type a0 = load_vec(h0 + i0, true), a1 = load_vec(h1 + i0, two);
+            typename Vec<T>::type b[CT];
+#pragma unroll
+            for (int q = 0; q < CT; q++)
+                b[q] = load_vec(y.P + ((size_t)r * R + 16 * q + cl) * n + i0, 16 * q + cl < R);
+            double top = 0.0;
+            if constexpr (STATS)
+#pragma unroll
+                for (int u = 0; u < VE; u++)
+                    top = fmax(top, fmax((double)fabs(Vec<T>::at(a0, u)), (double)fabs(Vec<T>::at(a1, u))));
+#pragma unroll
+            for (int q = 0; q < CT; q++)
+#pragma unroll
+                for (int u = 0; u < VE; u++) acc[0][q][u] = mma(Vec<T>::at(a0, u), Vec<T>::at(b[q], u), acc[0][q][u]);
+            if (two)
+#pragma unroll
+                for (int q = 0; q < CT; q++)
+#pragma unroll
+                    for (int u = 0; u < VE; u++) acc[1][q][u] = mma(Vec<T>::at(a1, u), Vec<T>::at(b[q], u), acc[1][q][u]);
+            return top;
+        };
+        if constexpr (STATS) {
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                if (16 * g < n)
+#pragma unroll
+                    for (int j = 0; j < 16 / KC; j++) hmax[g] = fmax(hmax[g], step(16 / KC * g + j));
+        } else {
+            for (int j = 0; j < n / KC; j++) step(j);
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int k = 16 * p + acc_row<T>(i, kk);
+                if (k >= cnt) continue;
+                T *z = c.z + (size_t)row_at(c, l, tile.y + k) * c.ZW + l * R;
+#pragma unroll
+                for (int q = 0; q < CT; q++) {
+                    T v;
+                    if constexpr (VE == 4) v = (acc[p][q][0][i] + acc[p][q][1][i]) + (acc[p][q][2][i] + acc[p][q][3][i]);
+                    else v = acc[p][q][0][i] + acc[p][q][1][i];
+                    if (16 * q + cl < R) z[16 * q + cl] = v;
+                    if constexpr (STATS) rmax[q] = fmax(rmax[q], (double)fabs(v));
+                }
+            }
+    }
+    if constexpr (STATS) {
+        double *st = c.stats + (size_t)l * (3 + n / 16 + R), top = 0.0;
+#pragma unroll
+        for (int g = 0; g < G; g++)
+            if (16 * g < n) {
+                max_into(st + 3 + g, hmax[g], lane);
+                top = fmax(top, hmax[g]);
+            }
+        max_into(st, top, lane);
+        top = 0.0;
+#pragma unroll
+        for (int q = 0; q < CT; q++) {
+            // the maximum of column cl over the four lane groups
+            double v = fmax(rmax[q], __shfl_xor(rmax[q], 16));
+            v = fmax(v, __shfl_xor(v, 32));
+            double *p = st + 3 + n / 16 + 16 * q + cl;
+            if (kk == 0 && 16 * q + cl < R && v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax((unsigned long long *)p, (unsigned long long)__double_as_longlong(v));
+            if (16 * q + cl < R) top = fmax(top, v);
+        }
+        max_into(st + 2, top, lane);
+    }
+}
+
+// logits = bias + sum over the layers of Q z: 32 consecutive rows per workgroup, a wavefront per 16 VE classes (VEC: the
+// classes are whole 16-byte vectors of the logits and of Q)
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void fl_logits(const FloatDevModel<T> m, const Chunk<T> c) {
+    constexpr int VE = kVE<T>, KC = 4 * VE;
+    const int C = m.classes, LR = m.L * m.R, lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
+    const T *Q = m.layers[0].Q;
+    const int r0 = blockIdx.x * 32;
+    for (int c0 = (threadIdx.x >> 6) * 16 * VE; c0 < C; c0 += 4 * 16 * VE) {
+        // class of component q: adjacent ones with VEC, else 16 apart
+        const int col = VEC ? c0 + VE * cl : c0 + cl, step = VEC ? 1 : 16;
+        // (two chains of additions per sum, joined with the bias last)
+        typename Acc<T>::type acc[2][2][VE];
+        T bias[VE];
+#pragma unroll
+        for (int q = 0; q < VE; q++) {
+            bias[q] = load_or_zero(m.output_bias + col + q * step, col + q * step < C);
+            for (int p = 0; p < 2; p++) acc[p][0][q] = acc[p][1][q] = typename Acc<T>::type{};
+        }
+        const T *z0 = c.z + (size_t)(r0 + cl < c.N ? r0 + cl : 0) * c.ZW;
+        const T *z1 = c.z + (size_t)(r0 + 16 + cl < c.N ? r0 + 16 + cl : 0) * c.ZW;
+        for (int j = 0; j < c.ZW / KC; j++) {
+            const int k0 = KC * j + VE * kk;
+            typename Vec<T>::type a0 = load_vec(z0 + k0, true), a1 = load_vec(z1 + k0, true), b[VE];
+#pragma unroll
+            for (int u = 0; u < VE; u++) {
+                const bool kok = k0 + u < LR;
+                if (!kok) ((T *)&a0)[u] = ((T *)&a1)[u] = T(0);
+                b[u] = typename Vec<T>::type{};
+                if constexpr (VEC) {
+                    b[u] = load_vec(Q + (size_t)(k0 + u) * C + col, kok && col < C);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < VE; q++)
+                        ((T *)&b[u])[q] = load_or_zero(Q + (size_t)(k0 + u) * C + col + q * 16, kok && col + q * 16 < C);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < VE; u++)
+#pragma unroll
+                for (int q = 0; q < VE; q++) {
+                    acc[0][u & 1][q] = mma(Vec<T>::at(a0, u), Vec<T>::at(b[u], q), acc[0][u & 1][q]);
+                    acc[1][u & 1][q] = mma(Vec<T>::at(a1, u), Vec<T>::at(b[u], q), acc[1][u & 1][q]);
+                }
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int row = r0 + 16 * p + acc_row<T>(i, kk);
+                if (row >= c.N) continue;
+                const int s = row / c.Tc;
+                if (row - s * c.Tc >= c.len(s)) continue;
+                T *out = c.logits + c.token_at(row) * C + col;
+                if constexpr (VEC) {
+                    typename Vec<T>::type v;
+#pragma unroll
+                    for (int q = 0; q < VE; q++) ((T *)&v)[q] = bias[q] + (acc[p][0][q][i] + acc[p][1][q][i]);
+                    if (col < C) *(typename Vec<T>::type *)out = v;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < VE; q++)
+                        if (col + q * 16 < C) out[q * 16] = bias[q] + (acc[p][0][q][i] + acc[p][1][q][i]);
+                }
+            }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------ host side
+size_t up256(size_t v) { return (v + 255) / 256 * 256; }
+
+struct Plan {
+    int64_t fixed, per_row;      // workspace bytes besides the rows' and per row (arrays rounded up apart)
+    int E, ZLW, ZW;
+    bool can_sort;
+};
+
+template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B) {
+    Plan p{};
+    const int64_t leaves = m.L > 1 ? (int64_t)1 << m.D : 1;
+    p.E = (int)(leaves > m.V ? leaves : m.V);
+    p.can_sort = p.E <= kSortLeaves;
+    p.ZLW = (m.R2 + 15) / 16 * 16;
+    p.ZW = (m.L * m.R + 15) / 16 * 16;
+    p.per_row = (int64_t)sizeof(T) * ((int64_t)m.L * (m.n + p.ZLW) + p.ZW) + (int64_t)m.L * 12;
+    p.fixed = 256 * 16 + B * 4;
+    if (p.can_sort) {
+        p.per_row += (int64_t)m.L * 16 / kTile + 1;
+        p.fixed += (int64_t)m.L * p.E * (16 + 8);
+    }
+    return p;
+}
+
+// Calls of fewer than 4 tokens stay on the step kernel, and so do transition blocks other than 16. At 4 tokens of 1 / 16 /
+// 256 / 1024 streams (us, step kernel / this form): small 132/77, 134/84, 135/98, 531/177; medium 148/90, 151/95, 161/127,
+// 629/214; large 189/113, 193/148, 219/227, 837/387; at fewer tokens the launches cost more than they save.
+constexpr int kScanTokens = 4;
+constexpr int64_t kScratchCap = (int64_t)1 << 30;
+
+template <typename T> bool takes(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
+    return m.b == 16 && B > 0 && Tn >= kScanTokens;
+}
+
+template <typename T> int64_t scratch_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
+    if (!takes(m, B, Tn)) return 0;
+    const Plan p = plan_of(m, B);
+    const int64_t want = p.fixed + p.per_row * B * Tn, least = p.fixed + p.per_row * 64;
+    const int64_t cap = kScratchCap > least ? kScratchCap : least;
+    return (int64_t)up256(want < cap ? want : cap);
+}
+
+template <typename T, int EPL> void route_of(const FloatDevModel<T> &m, const Chunk<T> &c, int l, hipStream_t st) {
+    const dim3 grid((c.N + 15) / 16), wg(256);
+    if (m.F % kVE<T> == 0) hipLaunchKernelGGL((fl_route<T, EPL, kVE<T>>), grid, wg, 0, st, m, c, l);
+    else hipLaunchKernelGGL((fl_route<T, EPL, 1>), grid, wg, 0, st, m, c, l);
+}
+
+template <typename T>
+int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T *state, T *logits, int32_t *leaves,
+             double *stats, void *scratch, int64_t bytes, hipStream_t st) {
+    const Plan p = plan_of(m, B);
+    // a chunk's rows; whole calls where they fit, else runs of at least 128 tokens of as many streams as fit
+    const int64_t rows = (bytes - p.fixed) / p.per_row;
+    if (rows < 1) return fail(YGG_ERR_ARG, "float scratch of %lld bytes is too small", (long long)bytes);
+    int64_t Tc = Tn, Bc = B;
+    if ((int64_t)B * Tn > rows) {
+        Tc = rows / B > 128 ? rows / B : 128;
+        if (Tc > Tn) Tc = Tn;
+        if (Tc > rows) Tc = rows;
+        Bc = rows / Tc < B ? rows / Tc : B;
+    }
+    const int LR = m.L, width = m.F + (m.router_state ? m.n : 0);
+    for (int s0 = 0; s0 < B; s0 += (int)Bc)
+        for (int t0 = 0; t0 < Tn; t0 += (int)Tc) {
+            Chunk<T> c{};
+            c.tokens = tokens;
+            c.Tn = Tn;
+            c.s0 = s0;
+            c.Bc = (int)(B - s0 < Bc ? B - s0 : Bc);
+            c.t0 = t0;
+            c.Tc = (int)(Tn - t0 < Tc ? Tn - t0 : Tc);
+            c.N = c.Bc * c.Tc;
+            c.E = p.E;
+            c.ZLW = p.ZLW;
+            c.ZW = p.ZW;
+            // sorting pays once an expert has about two rows on average (a sort's launches against the experts' second
+            // reading)
+            c.sorted = p.can_sort && c.N >= 2 * p.E;
+            c.max_tiles = c.sorted ? c.N / kTile + p.E : 0;
+            c.state = state;
+            c.logits = logits;
+            c.leaves = leaves;
+            c.stats = stats;
+            uint8_t *w = (uint8_t *)scratch;
+            auto take = [&](size_t k) {
+                uint8_t *q = w;
+                w += up256(k);
+                return q;
+            };
+            const size_t N = (size_t)c.N;
+            c.stop = (int *)take((size_t)B * 4);
+            c.done = (int *)take((size_t)LR * 4);
+            c.ntiles = (int *)take((size_t)LR * 4);
+            if (c.sorted) {
+                c.count = (int *)take((size_t)LR * p.E * 4);
+                c.off = (int *)take((size_t)LR * p.E * 4);
+                c.tiles = (int4 *)take((size_t)LR * c.max_tiles * 16);
+                c.rank = (int *)take(N * LR * 4);
+                c.order = (int *)take(N * LR * 4);
+            }
+            c.leaf = (int *)take(N * LR * 4);
+            c.z = (T *)take(N * p.ZW * sizeof(T));
+            c.zl = (T *)take(N * LR * p.ZLW * sizeof(T));
+            c.h = (T *)take(N * LR * m.n * sizeof(T));
+            if (w - (uint8_t *)scratch > bytes) return fail(YGG_ERR_ARG, "float scratch of %lld bytes is too small", (long long)bytes);
+            auto sort = [&](int l0, int layers) {
+                hipLaunchKernelGGL(fl_rank<T>, dim3((c.N + kRankRows - 1) / kRankRows, layers), dim3(1024),
+                                   p.E * sizeof(int), st, m, c, l0);
+                hipLaunchKernelGGL(fl_scatter<T>, dim3((c.N + 255) / 256, layers), dim3(256), 0, st, c, l0);
+            };
+            auto scan = [&](int l) {
+                constexpr int PD = sizeof(T) == 4 ? 8 : 5;
+                const dim3 grid((c.Bc + 3) / 4 * (m.n / 16));
+                if (l) hipLaunchKernelGGL((fl_scan<T, PD, false>), grid, dim3(64), 0, st, m, c, l);
+                else hipLaunchKernelGGL((fl_scan<T, PD, true>), grid, dim3(64), 0, st, m, c, l);
+            };
+            hipLaunchKernelGGL(fl_begin<T>, dim3((c.Bc + 3) / 4), dim3(256), 0, st, m, c);
+            scan(0);
+            for (int l = 1; l < m.L; l++) {
+                if (width <= 128) route_of<T, 8>(m, c, l, st);
+                else if (width <= 192) route_of<T, 12>(m, c, l, st);
+                else if (width <= 320) route_of<T, 20>(m, c, l, st);
+                else route_of<T, 32>(m, c, l, st);
+                if (c.sorted) sort(l == 1 ? 0 : l, l == 1 ? 2 : 1);
+                const int64_t waves = (int64_t)(c.sorted ? c.max_tiles : c.N) * ((m.n + 16 * kVE<T> - 1) / (16 * kVE<T>));
+                const int64_t wgs = (waves + 3) / 4;
+                hipLaunchKernelGGL(fl_input<T>, dim3((unsigned)(wgs < 8192 ? wgs : 8192)), dim3(256), 0, st, m, c, l);
+                scan(l);
+            }
+            if (m.L == 1 && c.sorted) sort(0, 1);
+            if (logits || stats) {
+                const int64_t wgs = ((int64_t)(c.sorted ? c.max_tiles : c.N) + 3) / 4, most = stats ? 1024 : 8192;
+                const dim3 grid((unsigned)(wgs < most ? wgs : most), m.L);
+                auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, m, c); };
+                if (m.R <= 16) stats ? go(fl_readout<T, 1, true>) : go(fl_readout<T, 1, false>);
+                else if (m.R <= 32) stats ? go(fl_readout<T, 2, true>) : go(fl_readout<T, 2, false>);
+                else stats ? go(fl_readout<T, 4, true>) : go(fl_readout<T, 4, false>);
+            }
+            if (logits) {
+                // 16-byte stores where every row of logits starts on 16 bytes
+                const bool vec = m.classes % kVE<T> == 0 && (uintptr_t)logits % 16 == 0;
+                const dim3 grid((c.N + 31) / 32);
+                if (vec) hipLaunchKernelGGL((fl_logits<T, true>), grid, dim3(256), 0, st, m, c);
+                else hipLaunchKernelGGL((fl_logits<T, false>), grid, dim3(256), 0, st, m, c);
+            }
+        }
+    HIP_TRY(hipGetLastError());
+    return YGG_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t ygg_float_scratch(const ygg_fmodel *m, int B, int T) {
+    if (!m || B < 0 || T < 0) return 0;
+    return m->precision == 32 ? scratch_of(m->m32, B, T) : scratch_of(m->m64, B, T);
+}
+
+int ygg_float_run_scratch(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, void *d_state, void *d_logits,
+                          int32_t *d_leaves, double *d_stats, void *d_scratch, int64_t scratch_bytes, void *stream) {
+    if (!m) return fail(YGG_ERR_ARG, "model is NULL");
+    if (B < 0 || T < 0) return fail(YGG_ERR_ARG, "negative B (%d) or T (%d)", B, T);
+    if (ygg_float_scratch(m, B, T) == 0)
+        return ygg_float_run(m, d_tokens, B, T, d_state, d_logits, d_leaves, d_stats, stream);
+    if (!d_state || !d_tokens) return fail(YGG_ERR_ARG, "tokens or state is NULL");
+    if (!d_scratch || (uintptr_t)d_scratch % 256) return fail(YGG_ERR_ARG, "scratch is NULL or not on 256 bytes");
+    DeviceGuard g;
+    HIP_TRY(g.set(m->device));
+    if (m->precision == 32)
+        return scan_run(m->m32, d_tokens, B, T, (float *)d_state, (float *)d_logits, d_leaves, d_stats, d_scratch,
+                        scratch_bytes, (hipStream_t)stream);
+    return scan_run(m->m64, d_tokens, B, T, (double *)d_state, (double *)d_logits, d_leaves, d_stats, d_scratch,
+                    scratch_bytes, (hipStream_t)stream);
+}
+
+}  // extern "C"

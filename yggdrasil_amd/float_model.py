@@ -307,7 +307,17 @@ class FloatYggdrasil:
         lg = torch.empty(B, T, self.classes, dtype=self.dtype, device=self.device) if logits else None
         lv = torch.empty(B, T, self.layers, dtype=torch.int32, device=self.device) if leaves else None
         sv = torch.zeros(self.layers, self.stats_stride, dtype=torch.float64, device=self.device) if stats else None
-        check(_lib.lib().ygg_float_run(self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(sv), _stream()))
+        lib, args = _lib.lib(), (self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(sv))
+        scratch, need = None, lib.ygg_float_scratch(self._h, B, T) if T > 1 else 0
+        if need:
+            try:
+                scratch = torch.empty(need, dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:      # the call without scratch still runs, token by token
+                pass
+        if scratch is None:
+            check(lib.ygg_float_run(*args, _stream()))
+        else:
+            check(lib.ygg_float_run_scratch(*args, _ptr(scratch), need, _stream()))
         e = ctypes.c_uint32()
         out = {"state": st}
         for k, v in (("logits", lg), ("leaves", lv), ("stats", sv)):
