@@ -146,6 +146,20 @@ int ygg_softmax(const float *d_logits, int64_t rows, int V, float *d_probs, floa
 int ygg_score(const ygg_model *m, const int32_t *d_tokens, const int32_t *d_targets, int B, int T, int8_t *d_state,
               double *d_nll, void *stream);
 
+/* ygg_run (without d_states and d_digest) and ygg_score layer by layer over the whole call instead of token by token:
+   all tokens are known, so only the transition inside a layer is sequential, and an expert's other weights are read once
+   for all the rows that take it. The same arguments and results, bit for bit; no counterpart in the reference. d_scratch:
+   device memory of scratch_bytes, 256-byte aligned, that no other call uses until this one has run. ygg_scratch gives
+   the bytes a call wants (score: of ygg_score_scratch; at most 512 MiB or 64 rows' worth; with less the call goes in more
+   and shorter chunks), or 0 where the token-by-token call is the faster or the only one: the two calls then take that way
+   and need no scratch. Environment, read at load: YGG_SCAN=0 never, YGG_SCAN=1 every call of at least 2 tokens (of the shapes
+   that have it), YGG_SCAN=sort the same with the rows always grouped by expert. */
+int64_t ygg_scratch(const ygg_model *m, int B, int T, int score);
+int ygg_run_scratch(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d_state, float *d_logits,
+                    int32_t *d_leaves, void *d_scratch, int64_t scratch_bytes, void *stream);
+int ygg_score_scratch(const ygg_model *m, const int32_t *d_tokens, const int32_t *d_targets, int B, int T,
+                      int8_t *d_state, double *d_nll, void *d_scratch, int64_t scratch_bytes, void *stream);
+
 /* Sample n tokens for each of B streams in one launch, every sampled token fed straight back as the next input: the
    generate loop of yggdrasil/inference.py:190-202 (and yggdrasil/inference_triton.py:229-248) after its prompt.
    Step t consumes x_t (x_0 = d_first[b], then x_t = d_out[b, t-1]) from d_state and samples d_out[b, t] from its

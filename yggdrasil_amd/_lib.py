@@ -15,7 +15,8 @@ LIB_PATH = Path(__file__).resolve().parent / "libygg_hip.so"
 
 # every entry point of include/ygg_hip.h
 SYMBOLS = ("ygg_load", "ygg_load_blob", "ygg_model_info", "ygg_free", "ygg_step", "ygg_run", "ygg_run_grouped",
-           "ygg_run_grouped_noalloc", "ygg_softmax", "ygg_score",
+           "ygg_run_grouped_noalloc", "ygg_softmax", "ygg_score", "ygg_scratch", "ygg_run_scratch",
+           "ygg_score_scratch",
            "ygg_generate", "ygg_take_errors", "ygg_float_load", "ygg_float_run", "ygg_float_scratch",
            "ygg_float_run_scratch", "ygg_float_take_errors",
            "ygg_float_free", "ygg_kernel_name", "ygg_spec_stats", "ygg_last_error", "ygg_version")
@@ -76,6 +77,10 @@ def lib() -> ctypes.CDLL:
     L.ygg_run.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp, vp]
     L.ygg_run_grouped.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp, vp]
     L.ygg_run_grouped_noalloc.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp, vp]
+    L.ygg_scratch.argtypes = [vp, i32, i32, i32]
+    L.ygg_scratch.restype = ctypes.c_int64
+    L.ygg_run_scratch.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, ctypes.c_int64, vp]
+    L.ygg_score_scratch.argtypes = [vp, vp, vp, i32, i32, vp, vp, vp, ctypes.c_int64, vp]
     L.ygg_softmax.argtypes = [vp, ctypes.c_int64, i32, vp, vp, vp]
     L.ygg_score.argtypes = [vp, vp, vp, i32, i32, vp, vp, vp]
     L.ygg_generate.argtypes = [vp, vp, i32, i32, vp, ctypes.c_float, i32, ctypes.c_uint64, vp, vp, vp]

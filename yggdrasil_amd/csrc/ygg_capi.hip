@@ -18,6 +18,7 @@
 
 #include "../../include/ygg_hip.h"
 #include "ygg_launch.h"
+#include "ygg_scan.h"
 #include "ygg_layout.h"
 
 namespace {
@@ -354,6 +355,32 @@ bool transitions_split(const FileArrays &fa, const std::vector<FileLayer> &fl) {
     return ok;
 }
 
+// Does the layer-by-layer form's 16-bit input hold (csrc/ygg_scan.hip)? The transition term stays within 2^14 + 1 at shift
+// >= 12, and the factored input and the layer input, each at most scale x 128 x 128 x rank, stay below 2^29, so that the
+// step's 32-bit sums never wrap and a clamped input saturates as the whole one. (Group scales: in every routed layer.)
+bool inputs_bounded(const FileArrays &fa, const std::vector<FileLayer> &fl, bool group) {
+    if (fa.shift < 12 || fa.R2 < 4) return false;
+    const float most = 536870912.0f / (128.0f * 128.0f);
+    for (size_t l = 1; l < fl.size(); l++) {
+        const FileLayer &y = fl[l];
+        if (group && !y.r2b) return false;
+        float top = fabsf(y.scal[3]);
+        for (int i = 0; y.mulv && i < fa.n; i++) top = std::max(top, fabsf(y.mulv[i]));
+        if (!(top * (float)fa.R2 < most)) return false;
+        if (!y.vt) continue;
+        float mt = 0.0f, fs = 0.0f;
+        for (int i = 0; i < fa.n; i++) mt = std::max(mt, fabsf(y.mT[i]));
+        for (int64_t e = 0; e < ((int64_t)1 << fa.D); e++) {
+            float v;
+            memcpy(&v, y.rec + e * y.record_bytes + y.off_S, 4);
+            if (!(fabsf(v) < 1e30f)) return false;
+            fs = std::max(fs, fabsf(v));
+        }
+        if (!(fs * mt * (float)fa.K < most)) return false;
+    }
+    return true;
+}
+
 // File record of one expert -> its gather record (layout in ygg_layout.h). split: A16 rows as hi bytes then lo bytes.
 void relayout_expert(const FileArrays &fa, const FileLayer &fy, const GatherLayout &gl, bool routed, bool split,
                      const uint8_t *frec, uint8_t *g) {
@@ -458,6 +485,9 @@ struct ygg_model {
     mutable uint32_t spec_next = 1;   // the next call's first epoch (epoch 0 never occurs: a cleared unit is stale)
     mutable std::mutex spec_mu;
     int spec_helpers = 0;             // helper workgroups of a call: enough for every candidate token
+    bool scan_ok = false;             // the layer-by-layer form takes the model (ygg_run_scratch, ygg_score_scratch)
+    bool scan_all = false;            // YGG_SCAN=1 or sort: every call of at least 2 tokens
+    bool scan_sort = false;           // YGG_SCAN=sort: its rows always sorted by expert
     bool grouped_ok = false;          // the leaf-grouped step takes the model (ygg_run_grouped)
     void *grp_ws = nullptr;           // its workspace, grown to the largest call
     size_t grp_ws_bytes = 0;
@@ -747,6 +777,13 @@ int load_impl(const uint8_t *data, size_t size, int device, ygg_model **out) {
         const int reach = ygg::flow_split_build(n, R, R2f, L, md) ? 8 * cus : 2 * resident;
         m->flow_max_streams[md] = flowk ? (m->flow_all ? INT32_MAX : std::max(resident, reach)) : 0;
     }
+    // the layer-by-layer form: every shape of the specialised kernels' families, tables or factored, whose inputs' 32-bit
+    // sums cannot wrap (YGG_SCAN=0: off, 1: every call of at least 2 tokens, sort: and their rows always sorted; off where
+    // another kernel is forced)
+    const char *scenv = getenv("YGG_SCAN");
+    m->scan_ok = family && L > 1 && kmode == "" && !(scenv && !strcmp(scenv, "0")) && inputs_bounded(fa, fl, group);
+    m->scan_sort = m->scan_ok && E <= 16384 && scenv && !strcmp(scenv, "sort");
+    m->scan_all = m->scan_sort || (m->scan_ok && scenv && !strcmp(scenv, "1"));
     // the leaf-grouped step: the benchmark shape with the specialised kernels' record layout, tensor scales, tables
     m->grouped_ok = family && !factored && !group && n == 128 && R == 8 && R2f == 16 && fa.blk == 16 &&
                     (L == 1 || fa.D <= 14);
@@ -874,6 +911,13 @@ const ygg::Kernel &pick(const ygg_model *m, int B, int T, int mode) {
 }
 
 
+// The calls the layer-by-layer form takes.
+bool scan_takes(const ygg_model *m, int B, int T) {
+    if (!m->scan_ok || B < 1 || T < 2) return false;
+    return m->scan_all || ygg::scan_pays(m->dev, B, T);
+}
+constexpr int64_t kScanScratchCap = (int64_t)1 << 29;
+
 }  // namespace
 
 namespace ygg {
@@ -956,6 +1000,50 @@ int ygg_run(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d
     io.states = d_states;
     io.digest = (unsigned long long *)d_digest;
     HIP_TRY(k.fn(m->dev, d_tokens, B, T, d_state, io, (hipStream_t)stream));
+    return YGG_OK;
+}
+
+int64_t ygg_scratch(const ygg_model *m, int B, int T, int score) {
+    if (!m || !scan_takes(m, B, T)) return 0;
+    return ygg::scan_scratch_bytes(m->dev, B, T, score != 0, m->scan_sort, kScanScratchCap);
+}
+
+int ygg_run_scratch(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d_state, float *d_logits,
+                    int32_t *d_leaves, void *d_scratch, int64_t scratch_bytes, void *stream) {
+    if (!m) return fail(YGG_ERR_ARG, "model is NULL");
+    if (B < 0 || T < 0) return fail(YGG_ERR_ARG, "negative B (%d) or T (%d)", B, T);
+    if (!scan_takes(m, B, T))
+        return ygg_run(m, d_tokens, B, T, d_state, d_logits, d_leaves, nullptr, nullptr, stream);
+    if (!d_state || !d_tokens) return fail(YGG_ERR_ARG, "tokens or state is NULL");
+    if (!d_scratch || (uintptr_t)d_scratch % 256) return fail(YGG_ERR_ARG, "scratch is NULL or not on 256 bytes");
+    if (scratch_bytes < ygg::scan_scratch_bytes(m->dev, B, 1, false, m->scan_sort, 0))
+        return fail(YGG_ERR_ARG, "scratch of %lld bytes is too small", (long long)scratch_bytes);
+    DeviceGuard g;
+    HIP_TRY(g.set(m->device));
+    YggIO io{};
+    io.logits = d_logits;
+    io.leaves = d_leaves;
+    HIP_TRY(ygg::launch_scan(m->dev, d_tokens, B, T, d_state, io, m->info.group != 0, m->scan_sort, d_scratch, scratch_bytes,
+                             (hipStream_t)stream));
+    return YGG_OK;
+}
+
+int ygg_score_scratch(const ygg_model *m, const int32_t *d_tokens, const int32_t *d_targets, int B, int T,
+                      int8_t *d_state, double *d_nll, void *d_scratch, int64_t scratch_bytes, void *stream) {
+    if (!m) return fail(YGG_ERR_ARG, "model is NULL");
+    if (B < 0 || T < 0) return fail(YGG_ERR_ARG, "negative B (%d) or T (%d)", B, T);
+    if (!scan_takes(m, B, T)) return ygg_score(m, d_tokens, d_targets, B, T, d_state, d_nll, stream);
+    if (!d_state || !d_nll || !d_tokens || !d_targets) return fail(YGG_ERR_ARG, "NULL buffer");
+    if (!d_scratch || (uintptr_t)d_scratch % 256) return fail(YGG_ERR_ARG, "scratch is NULL or not on 256 bytes");
+    if (scratch_bytes < ygg::scan_scratch_bytes(m->dev, B, 1, true, m->scan_sort, 0))
+        return fail(YGG_ERR_ARG, "scratch of %lld bytes is too small", (long long)scratch_bytes);
+    DeviceGuard g;
+    HIP_TRY(g.set(m->device));
+    YggIO io{};
+    io.targets = d_targets;
+    io.nll = d_nll;
+    HIP_TRY(ygg::launch_scan(m->dev, d_tokens, B, T, d_state, io, m->info.group != 0, m->scan_sort, d_scratch, scratch_bytes,
+                             (hipStream_t)stream));
     return YGG_OK;
 }
 

@@ -4,8 +4,8 @@
 // the route, the layer input, the expert's own input u = T_r[x] + U'_r (V' rms(h_below)) and the readout of a token need
 // nothing of the token before it in the same layer. So each layer runs over all rows (stream, token) of a chunk:
 //   fl_route    leaf and layer input of every row; 16 rows per workgroup
-//   fl_rank,    counting sort of the rows by leaf, and its tiles of at most 32 rows of one expert
-//   fl_scatter
+//   rows_count, counting sort of the rows by leaf, and its tiles of at most 32 rows of one expert (ygg_rows.h)
+//   rows_plan, rows_scatter
 //   fl_input    u: per tile the product of its rows' layer inputs and the expert's U', on the f32 / f64 matrix cores,
 //               plus the table rows
 //   fl_scan     the recurrence: 16 lanes per stream and block, A_r loaded ahead by token
@@ -13,20 +13,22 @@
 // the layers' ranks). The rows of few tokens are not sorted (a tile is one row then).
 //
 // Measured against the token-by-token kernel (whole calls, f32 unless said): 9 streams x 100 tokens of the medium
-// trained shape 3 635 -> 224 us; scoring 256 x 128 of the large one 6 597 -> 947; f64 calibration of 500 x 200 of the
-// medium one 45.6 -> 2.15 ms. The token-by-token kernel is bound by the dependent loads and barriers of a layer (7 us
+// trained shape 3 635 -> 173 us; scoring 256 x 128 of the large one 6 597 -> 939; f64 calibration of 500 x 200 of the
+// medium one 45.6 -> 2.0 ms. The token-by-token kernel is bound by the dependent loads and barriers of a layer (7 us
 // each), this form by its launches (17 to 26 of 4 us) at a thousand rows and by the experts' bytes at tens of thousands.
 #include <cstdlib>
+#include <type_traits>
 
 #include "ygg_float.h"
+#include "ygg_rows.h"
 
 using namespace ygg::flt;
+using namespace ygg::rows;
 
 namespace {
 
-constexpr int kTile = 32;            // rows of a tile of one expert (two 16-row matrix tiles)
-constexpr int kRankRows = 2048;      // rows of one counting-sort workgroup
-constexpr int kSortLeaves = 8192;    // most experts of a layer the sort's LDS histogram holds
+// A scan's wavefront loads this many rows past a stream's last without a look (tokens ahead and a run of them).
+constexpr int kPad = 64;
 
 template <typename T> struct Vec;    // the 16-byte vector of T
 template <> struct Vec<float> {
@@ -52,12 +54,12 @@ template <typename T> __device__ __forceinline__ int acc_row(int i, int q) { ret
 
 // v moved across lanes by a DPP control (both halves of a double)
 template <int CTRL> __device__ __forceinline__ float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 template <int CTRL> __device__ __forceinline__ double dpp(double v) {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 // the sum over aligned groups of 16 lanes, in every lane
@@ -80,21 +82,15 @@ template <typename T> __device__ __forceinline__ typename Vec<T>::type load_vec(
 template <typename T> struct Chunk {
     const int32_t *tokens;
     int Tn, s0, Bc, t0, Tc, N;
-    int E, ZLW, ZW, sorted, max_tiles;
+    int ZLW, ZW;
     T *state, *logits;
     int32_t *leaves;
     double *stats;
-    T *h;             // [L][N][n]: u, then the states
+    T *h;             // [L][N][n] (and kPad rows): u, then the states
     T *zl;            // [L][N][ZLW]: layer inputs, zero past R2
     T *z;             // [N][ZW]: readouts, layer l's at l R
-    int *leaf;        // [L][N], -1 past a stream's end
-    int *rank;        // [L][N] place of a row among its leaf's
-    int *order;       // [L][N] rows by leaf
-    int4 *tiles;      // [L][max_tiles]: leaf, first place in order, rows
-    int *ntiles;      // [L]
-    int *count;       // [L][E] rows per leaf
-    int *off;         // [L][E] a leaf's first place in order
-    int *done;        // [L] finished workgroups of fl_rank
+    Sort by[YGG_MAX_LAYERS];      // the rows of each layer by expert
+    int *r;           // [N + kPad] experts of the current layer's rows, 0 past a stream's end
     int *stop;        // [Bc] a stream's first token outside [0, V), or Tn
 
     __device__ __forceinline__ int len(int s) const {     // rows of stream s this chunk computes
@@ -107,46 +103,34 @@ template <typename T> struct Chunk {
     }
 };
 
-// a tile's leaf, first place and rows, or no rows; unsorted rows are tiles of one (i the same in the whole wavefront)
-template <typename T> __device__ __forceinline__ int4 tile_at(const Chunk<T> &c, int l, int i) {
-    int4 t;
-    if (c.sorted) {
-        t = c.tiles[(size_t)l * c.max_tiles + i];
-    } else {
-        const int r = c.leaf[(size_t)l * c.N + i];
-        t = make_int4(r, i, r >= 0 ? 1 : 0, 0);
-    }
-    return make_int4(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y),
-                     __builtin_amdgcn_readfirstlane(t.z), 0);
-}
-template <typename T> __device__ __forceinline__ int row_at(const Chunk<T> &c, int l, int place) {
-    return c.sorted ? c.order[(size_t)l * c.N + place] : place;
-}
-
-// Per stream (a wavefront) its end in this chunk, and layer 0's leaves (the tokens); the sort's counters cleared. The
+// Per stream (a workgroup) its end in this chunk, and layer 0's leaves (the tokens); the sort's counters cleared. The
 // streams' ends carry over to the next chunk.
 template <typename T> __global__ __launch_bounds__(256) void fl_begin(const FloatDevModel<T> m, const Chunk<T> c) {
-    const int lane = threadIdx.x & 63, s = (blockIdx.x * 256 + threadIdx.x) >> 6;
-    if (c.sorted)
-        for (int i = blockIdx.x * 256 + threadIdx.x; i < m.L * c.E; i += gridDim.x * 256) c.count[i] = 0;
-    if (blockIdx.x == 0 && threadIdx.x < m.L) c.done[threadIdx.x] = 0;
-    if (s >= c.Bc) return;
-    int stop = c.t0 ? c.stop[s] : c.Tn;
-    const int32_t *tok = c.tokens + (size_t)(c.s0 + s) * c.Tn + c.t0;
-    for (int t = 0; t < c.Tc; t += 64) {
-        const int x = t + lane < c.Tc ? tok[t + lane] : 0;
-        const unsigned long long bad = __ballot(x < 0 || x >= m.V);
-        if (bad && c.t0 + t < stop) {
-            stop = c.t0 + t + __builtin_ctzll(bad);
-            if (lane == 0) atomicOr(m.err, 1u);
-        }
-        if (t + lane < c.Tc) {
-            const bool live = c.t0 + t + lane < stop;
-            c.leaf[(size_t)s * c.Tc + t + lane] = live ? x : -1;
-            if (live && c.leaves) c.leaves[((size_t)(c.s0 + s) * c.Tn + c.t0 + t + lane) * m.L] = x;
-        }
+    __shared__ int first;
+    const int tid = threadIdx.x, s = blockIdx.x;
+    for (int l = 0; l < m.L && s == 0; l++) sort_clear(c.by[l]);
+    if (s == 0 && tid < kPad) c.r[c.N + tid] = 0;
+    const int was = c.t0 ? c.stop[s] : c.Tn;
+    if (tid == 0) first = was;
+    __syncthreads();
+    const size_t at = (size_t)(c.s0 + s) * c.Tn + c.t0, row0 = (size_t)s * c.Tc;
+    for (int t = tid; t < c.Tc; t += 256) {
+        const int x = c.tokens[at + t];
+        if (x < 0 || x >= m.V) atomicMin(&first, c.t0 + t);
     }
-    if (lane == 0) c.stop[s] = stop;
+    __syncthreads();
+    const int stop = first;
+    if (tid == 0) {
+        c.stop[s] = stop;
+        if (stop < was) atomicOr(m.err, 1u);
+    }
+    for (int t = tid; t < c.Tc; t += 256) {
+        const int x = c.tokens[at + t];
+        const bool live = c.t0 + t < stop;
+        c.by[0].leaf[row0 + t] = live ? x : -1;
+        c.r[row0 + t] = live ? x : 0;
+        if (live && c.leaves) c.leaves[(at + t) * m.L] = x;
+    }
 }
 
 // The route of layer l and its layer input: 16 rows per workgroup, 16 lanes per row. The descent reads one node row per
@@ -221,11 +205,12 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
         }
         if (rl == 0) {
             const int r = node - ((1 << m.D) - 1);
-            c.leaf[(size_t)l * c.N + row] = r;
+            c.by[l].leaf[row] = c.r[row] = r;
             if (c.leaves) c.leaves[at * m.L + l] = r;
         }
     } else if (row < c.N && rl == 0) {
-        c.leaf[(size_t)l * c.N + row] = -1;
+        c.by[l].leaf[row] = -1;
+        c.r[row] = 0;
     }
     if (!y.Vd) return;
     const int R2 = m.R2, kk = lane >> 4, cl = lane & 15;
@@ -268,79 +253,6 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
     }
 }
 
-// The counting sort's first half, for layers l0 + blockIdx.y: each workgroup counts its rows' leaves in LDS, takes the
-// leaves' places by one device-wide addition per leaf it saw (a leaf that most rows take costs one per workgroup, not
-// one per row), and the last workgroup to finish sums the counts into the leaves' first places and writes the tiles.
-template <typename T> __global__ __launch_bounds__(1024) void fl_rank(const FloatDevModel<T> m, const Chunk<T> c, int l0) {
-    extern __shared__ int hist[];
-    __shared__ int wsum[16][2], last;
-    const int l = l0 + blockIdx.y, tid = threadIdx.x, E = l == 0 ? m.V : 1 << m.D;
-    const int *leaf = c.leaf + (size_t)l * c.N;
-    int *count = c.count + (size_t)l * c.E, *off = c.off + (size_t)l * c.E;
-    for (int e = tid; e < E; e += 1024) hist[e] = 0;
-    __syncthreads();
-    constexpr int PER = kRankRows / 1024;
-    int lf[PER], at[PER];
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        const int row = blockIdx.x * kRankRows + k * 1024 + tid;
-        lf[k] = row < c.N ? leaf[row] : -1;
-        at[k] = lf[k] >= 0 ? atomicAdd(&hist[lf[k]], 1) : 0;
-    }
-    __syncthreads();
-    for (int e = tid; e < E; e += 1024)
-        if (hist[e]) hist[e] = __hip_atomic_fetch_add(&count[e], hist[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < PER; k++)
-        if (lf[k] >= 0) c.rank[(size_t)l * c.N + blockIdx.x * kRankRows + k * 1024 + tid] = hist[lf[k]] + at[k];
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) {
-        const int before = __hip_atomic_fetch_add(&c.done[l], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        last = before == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    // exclusive sums of the counts and of the tiles, each thread a run of leaves
-    const int per = (E + 1023) / 1024, e0 = tid * per;
-    int rows = 0, tl = 0;
-    for (int e = e0; e < e0 + per && e < E; e++) {
-        const int k = __hip_atomic_load(&count[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        rows += k;
-        tl += (k + kTile - 1) / kTile;
-    }
-    const int lane = tid & 63, wave = tid >> 6;
-    int ir = rows, it = tl;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(ir, o), b = __shfl_up(it, o);
-        if (lane >= o) ir += a, it += b;
-    }
-    if (lane == 63) wsum[wave][0] = ir, wsum[wave][1] = it;
-    __syncthreads();
-    int pr = ir - rows, pt = it - tl, total = 0;
-    for (int w = 0; w < 16; w++) {
-        if (w < wave) pr += wsum[w][0], pt += wsum[w][1];
-        total += wsum[w][1];
-    }
-    int4 *tiles = c.tiles + (size_t)l * c.max_tiles;
-    for (int e = e0; e < e0 + per && e < E; e++) {
-        const int k = __hip_atomic_load(&count[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        off[e] = pr;
-        for (int q = 0; q < k; q += kTile) tiles[pt++] = make_int4(e, pr + q, k - q < kTile ? k - q : kTile, 0);
-        pr += k;
-    }
-    if (tid == 0) c.ntiles[l] = total;
-}
-
-template <typename T> __global__ __launch_bounds__(256) void fl_scatter(const Chunk<T> c, int l0) {
-    const int l = l0 + blockIdx.y;
-    const int row = blockIdx.x * 256 + threadIdx.x;
-    if (row >= c.N) return;
-    const int r = c.leaf[(size_t)l * c.N + row];
-    if (r >= 0) c.order[(size_t)l * c.N + c.off[(size_t)l * c.E + r] + c.rank[(size_t)l * c.N + row]] = row;
-}
-
 // the maximum of a non-negative v over the wavefront into *p (non-negative doubles order as their bit patterns; most
 // wavefronts find a larger one there and add nothing)
 __device__ __forceinline__ void max_into(double *p, double v, int lane) {
@@ -356,16 +268,16 @@ template <typename T> __global__ __launch_bounds__(256) void fl_input(const Floa
     const FloatLayerDev<T> &y = m.layers[l];
     const int n = m.n, R2 = m.R2, CG = (n + 16 * VE - 1) / (16 * VE);
     const int lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
-    const int total = (c.sorted ? c.ntiles[l] : c.N) * CG;
+    const int total = tiles_of(c.by[l]) * CG;
     double zmax = 0.0;      // (calibration) the largest layer input
     for (int w = blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += gridDim.x * 4) {
-        const int4 tile = tile_at(c, l, w / CG);
+        const int4 tile = tile_at(c.by[l], w / CG);
         const int r = tile.x, cnt = tile.z;
         if (cnt == 0) continue;
         const int col = (w % CG) * 16 * VE + VE * cl;
         const bool cok = col < n, two = cnt > 16;
         int rows[2];
-        for (int q = 0; q < 2; q++) rows[q] = row_at(c, l, tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
+        for (int q = 0; q < 2; q++) rows[q] = row_at(c.by[l], tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
         typename Acc<T>::type acc[2][VE];
 #pragma unroll
         for (int q = 0; q < VE; q++) acc[0][q] = acc[1][q] = typename Acc<T>::type{};
@@ -397,7 +309,7 @@ template <typename T> __global__ __launch_bounds__(256) void fl_input(const Floa
             for (int i = 0; i < 4; i++) {
                 const int p = 16 * q + acc_row<T>(i, kk);
                 if (p < cnt && cok) {
-                    const int row = row_at(c, l, tile.y + p);
+                    const int row = row_at(c.by[l], tile.y + p);
                     typename Vec<T>::type t = *(const typename Vec<T>::type *)(
                         y.table + ((size_t)r * m.V + c.tokens[c.token_at(row)]) * n + col);
 #pragma unroll
@@ -419,75 +331,83 @@ template <typename T, int J = 0> __device__ __forceinline__ void block_dot(const
 }
 
 // The recurrence of layer l, h(t) = u(t) + A_r(t) h(t - 1): 16 lanes per stream and block of 16 coordinates, four
-// streams of one block per wavefront, the next PD tokens' A rows and inputs loaded ahead and the leaves PD further. The
-// loads of a token past a stream's end are those of its last one, so that every load is issued in straight-line code and
-// nothing but the token's own use waits for it. Workgroup b takes block b % (n / 16): workgroups go to the XCDs in turn,
-// so where n / 16 divides or is a multiple of 8 an XCD meets (n / 16) / 8 blocks, or one, whose share of the layer's A
-// stays in its L2. Layer 0 (L0) takes its input from the table.
+// streams of one block per wavefront (past the last stream its duplicates, whose equal stores change nothing), the next PD
+// tokens' A rows and inputs loaded ahead and their experts PD further. Loads run past a stream's end without a look (the
+// rows behind it, or kPad more): what they bring is never used. A wavefront on a SIMD of its own issues an instruction
+// every 4 cycles, so a step is kept short: the factors h_j come as row broadcasts inside the multiply-adds. Workgroup b
+// takes block b % (n / 16): workgroups go to the XCDs in turn, so where n / 16 divides or is a multiple of 8 an XCD meets
+// (n / 16) / 8 blocks, or one, whose share of the layer's A stays in its L2. Layer 0 (L0) takes its input from the table.
 template <typename T, int PD, bool L0>
 __global__ __launch_bounds__(64) void fl_scan(const FloatDevModel<T> m, const Chunk<T> c, int l) {
     constexpr int VE = kVE<T>, CH = 16 / VE;
     const FloatLayerDev<T> &y = m.layers[l];
     const int n = m.n, nb = n / 16, g = blockIdx.x % nb, lane = threadIdx.x & 63, i = lane & 15;
     const int sw = blockIdx.x / nb * 4 + (lane >> 4), s = sw < c.Bc ? sw : c.Bc - 1;
-    const bool mine = sw < c.Bc;
-    const int len = c.len(s), last = len > 0 ? len - 1 : 0;
-    T *st = c.state + ((size_t)(c.s0 + s) * m.L + l) * n + g * 16 + i;
-    T *h = c.h + ((size_t)l * c.N + (size_t)s * c.Tc) * n + g * 16 + i;
-    const int *leaf = c.leaf + (size_t)l * c.N + (size_t)s * c.Tc;
-    // the most tokens any stream of the wavefront takes
-    int most = len;
+    const int len = c.len(s);
+    int most = len, least = len;          // the most and the fewest tokens of the wavefront's streams
     for (int o = 16; o < 64; o <<= 1) {
-        const int k = __shfl_xor(most, o);
-        most = k > most ? k : most;
+        const int a = __shfl_xor(most, o), b = __shfl_xor(least, o);
+        most = a > most ? a : most;
+        least = b < least ? b : least;
     }
     most = __builtin_amdgcn_readfirstlane(most);
+    least = __builtin_amdgcn_readfirstlane(least);
     if (most == 0) return;
+    T *st = c.state + ((size_t)(c.s0 + s) * m.L + l) * n + g * 16 + i;
+    T *h = c.h + ((size_t)l * c.N + (size_t)s * c.Tc) * n + g * 16 + i;
+    const int *rs = c.r + (size_t)s * c.Tc;
     const T *table = y.table + g * 16 + i;
+    T hv = *st;
     if (!y.A) {     // no recurrence
-        T hv = *st;
         for (int t = 0; t < len; t++) {
-            hv = L0 ? table[(size_t)leaf[t] * n] : h[(size_t)t * n];
-            if (L0 && mine) h[(size_t)t * n] = hv;
+            hv = L0 ? table[(size_t)rs[t] * n] : h[(size_t)t * n];
+            if (L0) h[(size_t)t * n] = hv;
         }
-        if (mine) *st = hv;
+        *st = hv;
         return;
     }
     const T *A = y.A + (size_t)g * 256 + VE * i;
-    T hv = *st;
+    const uint32_t stride = (uint32_t)nb * 256;      // entries of an expert's A
     typename Vec<T>::type a[PD][CH];
     T u[PD];
-    int lf[PD];
-    auto fetch = [&](typename Vec<T>::type (&av)[CH], T &uv, int lv, int t) {
-        const int r = lv > 0 ? lv : 0;      // (a stream that stops at once has no leaf)
-        const T *ab = A + (size_t)r * nb * 256;
+    int r[PD];
+    auto fetch = [&](int k, int d) {       // the token d rows on, whose expert is in r[k], into slot k
+        // (the expert is used here and no earlier: hoisted, its use waits for every load up to its own, PD tokens early)
+        asm volatile("" : "+v"(r[k]));
+        const T *ab = A + (uint64_t)(uint32_t)r[k] * stride;
 #pragma unroll
-        for (int k = 0; k < CH; k++) av[k] = *(const typename Vec<T>::type *)(ab + k * 16 * VE);
-        uv = L0 ? table[(size_t)r * n] : h[(size_t)(t < last ? t : last) * n];
+        for (int q = 0; q < CH; q++) a[k][q] = *(const typename Vec<T>::type *)(ab + q * 16 * VE);
+        u[k] = L0 ? table[(uint64_t)(uint32_t)r[k] * (uint32_t)n] : h[(size_t)(d * n)];
     };
 #pragma unroll
-    for (int k = 0; k < PD; k++) lf[k] = leaf[k < last ? k : last];
+    for (int k = 0; k < PD; k++) r[k] = rs[k];
+    // (in the loop's order: the waits at its top are those of the worse of the two ways in)
 #pragma unroll
-    for (int k = 0; k < PD; k++) fetch(a[k], u[k], lf[k], k);
-#pragma unroll
-    for (int k = 0; k < PD; k++) lf[k] = leaf[PD + k < last ? PD + k : last];
-    for (int t0 = 0; t0 < most; t0 += PD) {
+    for (int k = 0; k < PD; k++) {
+        fetch(k, k);
+        r[k] = rs[PD + k];
+    }
+    auto run = [&](auto tail, int left) {
 #pragma unroll
         for (int k = 0; k < PD; k++) {
-            const int t = t0 + k;
             T av[16], sums[4] = {T(0), T(0), T(0), T(0)};
 #pragma unroll
             for (int j = 0; j < 16; j++) av[j] = Vec<T>::at(a[k][j / VE], j % VE);
             block_dot<T>(av, hv, sums);
             const T hn = u[k] + ((sums[0] + sums[1]) + (sums[2] + sums[3]));
-            const bool on = t < len;
+            const bool on = !decltype(tail)::value || k < left;
             hv = on ? hn : hv;
-            if (on && mine) h[(size_t)t * n] = hv;
-            fetch(a[k], u[k], lf[k], t + PD);
-            lf[k] = leaf[t + 2 * PD < last ? t + 2 * PD : last];
+            if (on) h[(size_t)(k * n)] = hv;
+            fetch(k, k + PD);
+            r[k] = rs[k + 2 * PD];
         }
-    }
-    if (mine) *st = hv;
+        h += (size_t)(PD * n);
+        rs += PD;
+    };
+    int t0 = 0;
+    for (; t0 + PD <= least; t0 += PD) run(std::false_type(), PD);
+    for (; t0 < most; t0 += PD) run(std::true_type(), len - t0);
+    *st = hv;
 }
 
 // z = P_r h of every layer (blockIdx.y): a wavefront per tile; CT column tiles of 16 ranks, each summed in VE chains (a
@@ -499,17 +419,17 @@ __global__ __launch_bounds__(256) void fl_readout(const FloatDevModel<T> m, cons
     const int l = blockIdx.y;
     const FloatLayerDev<T> &y = m.layers[l];
     const int n = m.n, R = m.R, lane = threadIdx.x & 63, kk = lane >> 4, cl = lane & 15;
-    const int total = c.sorted ? c.ntiles[l] : c.N;
+    const int total = tiles_of(c.by[l]);
     double hmax[STATS ? G : 1], rmax[STATS ? CT : 1];
     for (double &v : hmax) v = 0.0;
     for (double &v : rmax) v = 0.0;
     for (int w = blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += gridDim.x * 4) {
-        const int4 tile = tile_at(c, l, w);
+        const int4 tile = tile_at(c.by[l], w);
         const int r = tile.x, cnt = tile.z;
         if (cnt == 0) continue;
         const bool two = cnt > 16;
         int rows[2];
-        for (int q = 0; q < 2; q++) rows[q] = row_at(c, l, tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
+        for (int q = 0; q < 2; q++) rows[q] = row_at(c.by[l], tile.y + (16 * q + cl < cnt ? 16 * q + cl : 0));
         const T *h0 = c.h + ((size_t)l * c.N + rows[0]) * n, *h1 = c.h + ((size_t)l * c.N + rows[1]) * n;
         typename Acc<T>::type acc[2][CT][VE];
 #pragma unroll
@@ -554,7 +474,7 @@ __global__ __launch_bounds__(256) void fl_readout(const FloatDevModel<T> m, cons
             for (int i = 0; i < 4; i++) {
                 const int k = 16 * p + acc_row<T>(i, kk);
                 if (k >= cnt) continue;
-                T *z = c.z + (size_t)row_at(c, l, tile.y + k) * c.ZW + l * R;
+                T *z = c.z + (size_t)row_at(c.by[l], tile.y + k) * c.ZW + l * R;
 #pragma unroll
                 for (int q = 0; q < CT; q++) {
                     T v;
@@ -658,27 +578,22 @@ __global__ __launch_bounds__(256) void fl_logits(const FloatDevModel<T> m, const
 }
 
 // ------------------------------------------------------------------------------------------------------ host side
-size_t up256(size_t v) { return (v + 255) / 256 * 256; }
+// Sorting pays once an expert has about two rows on average (the sort's launches against reading experts again)
+bool sort_pays(int64_t N, int E) { return E <= kSortLeaves && N >= 2 * (int64_t)E; }
 
 struct Plan {
     int64_t fixed, per_row;      // workspace bytes besides the rows' and per row (arrays rounded up apart)
     int E, ZLW, ZW;
-    bool can_sort;
 };
 
-template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B) {
+template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
     Plan p{};
     const int64_t leaves = m.L > 1 ? (int64_t)1 << m.D : 1;
     p.E = (int)(leaves > m.V ? leaves : m.V);
-    p.can_sort = p.E <= kSortLeaves;
     p.ZLW = (m.R2 + 15) / 16 * 16;
     p.ZW = (m.L * m.R + 15) / 16 * 16;
-    p.per_row = (int64_t)sizeof(T) * ((int64_t)m.L * (m.n + p.ZLW) + p.ZW) + (int64_t)m.L * 12;
-    p.fixed = 256 * 16 + B * 4;
-    if (p.can_sort) {
-        p.per_row += (int64_t)m.L * 16 / kTile + 1;
-        p.fixed += (int64_t)m.L * p.E * (16 + 8);
-    }
+    p.per_row = (int64_t)sizeof(T) * ((int64_t)m.L * (m.n + p.ZLW) + p.ZW) + 4 + m.L * kSortRowBytes;
+    p.fixed = 256 * 8 + B * 4 + kPad * (4 + (int64_t)m.n * sizeof(T)) + m.L * sort_fixed_bytes(B * Tn, p.E, sort_pays(B * Tn, p.E));
     return p;
 }
 
@@ -694,7 +609,7 @@ template <typename T> bool takes(const FloatDevModel<T> &m, int64_t B, int64_t T
 
 template <typename T> int64_t scratch_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
     if (!takes(m, B, Tn)) return 0;
-    const Plan p = plan_of(m, B);
+    const Plan p = plan_of(m, B, Tn);
     const int64_t want = p.fixed + p.per_row * B * Tn, least = p.fixed + p.per_row * 64;
     const int64_t cap = kScratchCap > least ? kScratchCap : least;
     return (int64_t)up256(want < cap ? want : cap);
@@ -709,7 +624,7 @@ template <typename T, int EPL> void route_of(const FloatDevModel<T> &m, const Ch
 template <typename T>
 int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T *state, T *logits, int32_t *leaves,
              double *stats, void *scratch, int64_t bytes, hipStream_t st) {
-    const Plan p = plan_of(m, B);
+    const Plan p = plan_of(m, B, Tn);
     // a chunk's rows; whole calls where they fit, else runs of at least 128 tokens of as many streams as fit
     const int64_t rows = (bytes - p.fixed) / p.per_row;
     if (rows < 1) return fail(YGG_ERR_ARG, "float scratch of %lld bytes is too small", (long long)bytes);
@@ -720,7 +635,7 @@ int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T 
         if (Tc > rows) Tc = rows;
         Bc = rows / Tc < B ? rows / Tc : B;
     }
-    const int LR = m.L, width = m.F + (m.router_state ? m.n : 0);
+    const int width = m.F + (m.router_state ? m.n : 0);
     for (int s0 = 0; s0 < B; s0 += (int)Bc)
         for (int t0 = 0; t0 < Tn; t0 += (int)Tc) {
             Chunk<T> c{};
@@ -731,13 +646,9 @@ int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T 
             c.t0 = t0;
             c.Tc = (int)(Tn - t0 < Tc ? Tn - t0 : Tc);
             c.N = c.Bc * c.Tc;
-            c.E = p.E;
             c.ZLW = p.ZLW;
             c.ZW = p.ZW;
-            // sorting pays once an expert has about two rows on average (a sort's launches against the experts' second
-            // reading)
-            c.sorted = p.can_sort && c.N >= 2 * p.E;
-            c.max_tiles = c.sorted ? c.N / kTile + p.E : 0;
+            const bool sorted = sort_pays(c.N, p.E);
             c.state = state;
             c.logits = logits;
             c.leaves = leaves;
@@ -750,47 +661,34 @@ int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T 
             };
             const size_t N = (size_t)c.N;
             c.stop = (int *)take((size_t)B * 4);
-            c.done = (int *)take((size_t)LR * 4);
-            c.ntiles = (int *)take((size_t)LR * 4);
-            if (c.sorted) {
-                c.count = (int *)take((size_t)LR * p.E * 4);
-                c.off = (int *)take((size_t)LR * p.E * 4);
-                c.tiles = (int4 *)take((size_t)LR * c.max_tiles * 16);
-                c.rank = (int *)take(N * LR * 4);
-                c.order = (int *)take(N * LR * 4);
-            }
-            c.leaf = (int *)take(N * LR * 4);
+            for (int l = 0; l < m.L; l++) lay_out(c.by[l], c.N, l ? 1 << m.D : m.V, sorted, take);
             c.z = (T *)take(N * p.ZW * sizeof(T));
-            c.zl = (T *)take(N * LR * p.ZLW * sizeof(T));
-            c.h = (T *)take(N * LR * m.n * sizeof(T));
+            c.zl = (T *)take(N * m.L * p.ZLW * sizeof(T));
+            c.r = (int *)take((N + kPad) * 4);
+            c.h = (T *)take((N * m.L + kPad) * m.n * sizeof(T));
             if (w - (uint8_t *)scratch > bytes) return fail(YGG_ERR_ARG, "float scratch of %lld bytes is too small", (long long)bytes);
-            auto sort = [&](int l0, int layers) {
-                hipLaunchKernelGGL(fl_rank<T>, dim3((c.N + kRankRows - 1) / kRankRows, layers), dim3(1024),
-                                   p.E * sizeof(int), st, m, c, l0);
-                hipLaunchKernelGGL(fl_scatter<T>, dim3((c.N + 255) / 256, layers), dim3(256), 0, st, c, l0);
-            };
             auto scan = [&](int l) {
                 constexpr int PD = sizeof(T) == 4 ? 8 : 5;
                 const dim3 grid((c.Bc + 3) / 4 * (m.n / 16));
                 if (l) hipLaunchKernelGGL((fl_scan<T, PD, false>), grid, dim3(64), 0, st, m, c, l);
                 else hipLaunchKernelGGL((fl_scan<T, PD, true>), grid, dim3(64), 0, st, m, c, l);
             };
-            hipLaunchKernelGGL(fl_begin<T>, dim3((c.Bc + 3) / 4), dim3(256), 0, st, m, c);
+            hipLaunchKernelGGL(fl_begin<T>, dim3(c.Bc), dim3(256), 0, st, m, c);
             scan(0);
             for (int l = 1; l < m.L; l++) {
                 if (width <= 128) route_of<T, 8>(m, c, l, st);
                 else if (width <= 192) route_of<T, 12>(m, c, l, st);
                 else if (width <= 320) route_of<T, 20>(m, c, l, st);
                 else route_of<T, 32>(m, c, l, st);
-                if (c.sorted) sort(l == 1 ? 0 : l, l == 1 ? 2 : 1);
-                const int64_t waves = (int64_t)(c.sorted ? c.max_tiles : c.N) * ((m.n + 16 * kVE<T> - 1) / (16 * kVE<T>));
+                if (sorted) launch_sort(c.by[l], c.by[0], l == 1, st);
+                const int64_t waves = (int64_t)(sorted ? c.by[l].max_tiles : c.N) * ((m.n + 16 * kVE<T> - 1) / (16 * kVE<T>));
                 const int64_t wgs = (waves + 3) / 4;
                 hipLaunchKernelGGL(fl_input<T>, dim3((unsigned)(wgs < 8192 ? wgs : 8192)), dim3(256), 0, st, m, c, l);
                 scan(l);
             }
-            if (m.L == 1 && c.sorted) sort(0, 1);
+            if (m.L == 1 && sorted) launch_sort(c.by[0], c.by[0], false, st);
             if (logits || stats) {
-                const int64_t wgs = ((int64_t)(c.sorted ? c.max_tiles : c.N) + 3) / 4, most = stats ? 1024 : 8192;
+                const int64_t wgs = ((int64_t)(sorted ? c.N / kTile + p.E : c.N) + 3) / 4, most = stats ? 1024 : 8192;
                 const dim3 grid((unsigned)(wgs < most ? wgs : most), m.L);
                 auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, m, c); };
                 if (m.R <= 16) stats ? go(fl_readout<T, 1, true>) : go(fl_readout<T, 1, false>);

@@ -131,10 +131,10 @@ __device__ __forceinline__ double exp_neg(double d, ConstF64 c) {
     return d < -745.5 ? 0.0 : ldexp(p, (int)k);
 }
 
-// Token t's term into acc: lg classes [4 lane, 4 lane + 4) of this lane, V classes; y is uniform and in range. The
-// sum over classes runs as a tree over lanes instead of in class order, so se can differ from the reference's in its
-// last bits.
-__device__ __forceinline__ void token_nll(NllSum &acc, const float (&lg)[4], int V, int y, int lane) {
+// A token's two terms, se and lin = mx - lg[y]: lg classes [4 lane, 4 lane + 4) of this lane, V classes; y is uniform and
+// in range. The sum over classes runs as a tree over lanes instead of in class order, so se can differ from the
+// reference's in its last bits.
+__device__ __forceinline__ void nll_terms(double &se, double &lin, const float (&lg)[4], int V, int y, int lane) {
     float mx = -__builtin_huge_valf();
 #pragma unroll
     for (int u = 0; u < 4; u++)
@@ -142,7 +142,7 @@ __device__ __forceinline__ void token_nll(NllSum &acc, const float (&lg)[4], int
     mx = wave_max_f32(mx);
     ConstF64 c = (ConstF64)kExpNeg;
     asm volatile("" : "+s"(c));
-    double se = 0.0;
+    se = 0.0;
 #pragma unroll
     for (int u = 0; u < 4; u++)
         if (4 * lane + u < V) se += exp_neg((double)lg[u] - (double)mx, c);
@@ -151,7 +151,12 @@ __device__ __forceinline__ void token_nll(NllSum &acc, const float (&lg)[4], int
 #pragma unroll
     for (int u = 1; u < 4; u++) ly = (y & 3) == u ? lg[u] : ly;
     ly = __shfl(ly, y >> 2);
-    acc.add(se, (double)mx - (double)ly);
+    lin = (double)mx - (double)ly;
+}
+__device__ __forceinline__ void token_nll(NllSum &acc, const float (&lg)[4], int V, int y, int lane) {
+    double se, lin;
+    nll_terms(se, lin, lg, V, y, lane);
+    acc.add(se, lin);
 }
 
 __device__ __forceinline__ float wave_sum_f32(float v) {

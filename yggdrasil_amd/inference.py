@@ -207,6 +207,17 @@ class Yggdrasil:
         g.replay()
         return logits.clone(), h.clone()
 
+    def _scratch(self, B: int, T: int, score: bool):
+        """(device scratch, its bytes) of a call that runs layer by layer over its known tokens (ygg_scratch), or
+        (None, 0) where it runs token by token: that is what the call takes, or there is no memory for the scratch."""
+        need = _lib.lib().ygg_scratch(self._h, B, T, int(score)) if T > 1 else 0
+        if not need:
+            return None, 0
+        try:
+            return torch.empty(need, dtype=torch.uint8, device=self.device), need
+        except torch.OutOfMemoryError:
+            return None, 0
+
     def run(self, tokens, state: Optional[torch.Tensor] = None, logits: bool = True, leaves: bool = False,
             states: bool = False, digest=False, _entry: str = "ygg_run") -> dict:
         """T tokens per stream in one launch: tokens (B, T) from state (default zero; not modified) ->
@@ -235,8 +246,14 @@ class Yggdrasil:
                             device=dev)
         else:
             dg = None
-        check(getattr(_lib.lib(), _entry)(self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(sv), _ptr(dg),
-                                          _stream()))
+        scratch, need = (None, 0) if sv is not None or dg is not None or _entry != "ygg_run" else \
+            self._scratch(B, T, False)
+        if scratch is not None:
+            check(_lib.lib().ygg_run_scratch(self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(scratch), need,
+                                             _stream()))
+        else:
+            check(getattr(_lib.lib(), _entry)(self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(sv), _ptr(dg),
+                                              _stream()))
         for k, v in (("logits", lg), ("leaves", lv), ("states", sv), ("digest", dg)):
             if v is not None:
                 out[k] = v
@@ -279,7 +296,12 @@ class Yggdrasil:
             nll = torch.zeros(B, dtype=torch.float64, device=self.device)
             if T > 0:
                 xd, yd = self._tokens(np.ascontiguousarray(xin)), self._tokens(np.ascontiguousarray(tgt))
-                check(_lib.lib().ygg_score(self._h, _ptr(xd), _ptr(yd), B, T, _ptr(st), _ptr(nll), _stream()))
+                scratch, need = self._scratch(B, T, True)
+                if scratch is not None:
+                    check(_lib.lib().ygg_score_scratch(self._h, _ptr(xd), _ptr(yd), B, T, _ptr(st), _ptr(nll),
+                                                       _ptr(scratch), need, _stream()))
+                else:
+                    check(_lib.lib().ygg_score(self._h, _ptr(xd), _ptr(yd), B, T, _ptr(st), _ptr(nll), _stream()))
             out.append((nll / LN2).cpu().numpy())
         return np.concatenate(out) if out else np.zeros(0)
 
