@@ -63,6 +63,7 @@ template <int CTRL> __device__ __forceinline__ float dpp_f32(float v) {
 __device__ __forceinline__ float lane_f32(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
+__device__ __forceinline__ unsigned long long lane_mask(bool pred) { return __builtin_amdgcn_ballot_w64(pred); }
 // fmaxf over the wavefront (every lane active), returned to every lane: DPP within rows of 16 lanes (quad swaps, the
 // half-row and row mirrors), then the four row maxima from scalar reads. fmaxf ignores NaNs and is exact, so the order
 // of the pairings does not change the result.
@@ -72,6 +73,18 @@ __device__ __forceinline__ float wave_max_f32(float v) {
     v = fmaxf(v, dpp_f32<0x141>(v));
     v = fmaxf(v, dpp_f32<0x140>(v));
     return fmaxf(fmaxf(lane_f32(v, 0), lane_f32(v, 16)), fmaxf(lane_f32(v, 32), lane_f32(v, 48)));
+}
+// the same of unsigned integers
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    auto step = [&](uint32_t w) { v = w > v ? w : v; };
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false));
+    const uint32_t a = __builtin_amdgcn_readlane((int)v, 0), b = __builtin_amdgcn_readlane((int)v, 16),
+                   c = __builtin_amdgcn_readlane((int)v, 32), d = __builtin_amdgcn_readlane((int)v, 48);
+    const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
+    return ab > cd ? ab : cd;
 }
 __device__ __forceinline__ double wave_sum_f64(double v) {
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
@@ -211,18 +224,27 @@ __device__ __forceinline__ int sample_token(const float (&lg)[4], int V, float t
         const int u = ((mk[0] >> ln) & 1) ? 0 : (((mk[1] >> ln) & 1) ? 1 : (((mk[2] >> ln) & 1) ? 2 : 3));
         return 4 * ln + u;
     }
-    // the top_k-th largest logit, by a radix search over order-preserving keys
+    // A key that exactly the classes of the top_k largest logits reach (with ties at the last of them, its own key), by a
+    // radix search over order-preserving keys. A token waits for every step of it, so a bit above the largest key is
+    // passed without a count, and the search ends where a count is top_k: from there on the set stays the same. (All 32
+    // bits counted took 3.4 us of a token's 9.2 at one stream of the medium trained shape.)
     uint32_t kth = 0;
     if (top_k > 0 && top_k < V) {
-        uint32_t key[4];
+        uint32_t key[4], most = 0;
 #pragma unroll
-        for (int u = 0; u < 4; u++) key[u] = fkey(lg[u]);
-        for (int b = 31; b >= 0; b--) {
+        for (int u = 0; u < 4; u++) {
+            key[u] = valid[u] ? fkey(lg[u]) : 0u;      // (no candidate is 0)
+            most = key[u] > most ? key[u] : most;
+        }
+        most = wave_max_u32(most);
+        for (int b = 31 - __builtin_clz(most | 1u); b >= 0; b--) {
             const uint32_t cand = kth | (1u << b);
+            if (cand > most) continue;
             int c = 0;     // classes with keys >= cand: population counts of ballots
 #pragma unroll
-            for (int u = 0; u < 4; u++) c += __popcll(__ballot(valid[u] && key[u] >= cand));
+            for (int u = 0; u < 4; u++) c += __popcll(lane_mask(key[u] >= cand));
             if (c >= top_k) kth = cand;
+            if (c == top_k) break;
         }
     }
     float w[4], part = 0.0f;
@@ -233,7 +255,7 @@ __device__ __forceinline__ int sample_token(const float (&lg)[4], int V, float t
         part += w[u];
     }
     const float incl = wave_scan_f32(part, lane);
-    const float total = __shfl(incl, 63);
+    const float total = lane_f32(incl, 63);
     const unsigned long long r = mix64(seed ^ mix64(((unsigned long long)s << 32) | (unsigned)t));
     const float target = (float)(r >> 40) * (1.0f / 16777216.0f) * total;
     // the first class whose running sum exceeds the target (the last kept class when rounding leaves none)
@@ -301,7 +323,6 @@ __device__ __forceinline__ int walk_bits(unsigned long long mask, int h) {
 }
 
 // the lanes whose pred holds, as a wavefront-uniform 64-bit mask
-__device__ __forceinline__ unsigned long long lane_mask(bool pred) { return __builtin_amdgcn_ballot_w64(pred); }
 
 // _mm512_cvtps_epi32 in round-to-nearest-even: NaN and |x| >= 2^31 give INT32_MIN (cpu/ygg.cpp:292 and others)
 __device__ __forceinline__ int cvt_rne(float x) {
