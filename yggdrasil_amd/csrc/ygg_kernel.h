@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     const uint32_t a = __builtin_amdgcn_readlane((int)v, 0), b = __builtin_amdgcn_readlane((int)v, 16),
                    c = __builtin_amdgcn_readlane((int)v, 32), d = __builtin_amdgcn_readlane((int)v, 48);
     const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
-    return ab > cd ? ab : cd;
+    return __builtin_amdgcn_readfirstlane((int)(ab > cd ? ab : cd));
 }
 __device__ __forceinline__ double wave_sum_f64(double v) {
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
@@ -226,8 +226,9 @@ __device__ __forceinline__ int sample_token(const float (&lg)[4], int V, float t
     }
     // A key that exactly the classes of the top_k largest logits reach (with ties at the last of them, its own key), by a
     // radix search over order-preserving keys. A token waits for every step of it, so a bit above the largest key is
-    // passed without a count, and the search ends where a count is top_k: from there on the set stays the same. (All 32
-    // bits counted took 3.4 us of a token's 9.2 at one stream of the medium trained shape.)
+    // passed without a count, and the search ends where a count is top_k: from there on the set stays the same. (At one
+    // stream of the medium trained shape, temperature 0.8 and top 20, a token took 9.20 us with all 32 bits counted and
+    // 6.7 with this loop of one branch and about 15 rounds; the same without top_k 5.74.)
     uint32_t kth = 0;
     if (top_k > 0 && top_k < V) {
         uint32_t key[4], most = 0;
@@ -237,15 +238,19 @@ __device__ __forceinline__ int sample_token(const float (&lg)[4], int V, float t
             most = key[u] > most ? key[u] : most;
         }
         most = wave_max_u32(most);
-        for (int b = 31 - __builtin_clz(most | 1u); b >= 0; b--) {
-            const uint32_t cand = kth | (1u << b);
-            if (cand > most) continue;
-            int c = 0;     // classes with keys >= cand: population counts of ballots
+        uint32_t bit = 0x80000000u;
+        int c;
+        do {
+            // while kth is a prefix of the largest key, the next bit that a key can have
+            const uint32_t rest = most ^ kth;
+            bit = rest >> 1 >= bit ? bit : 0x80000000u >> __builtin_clz(rest | 1u);
+            const uint32_t cand = kth | bit;
+            c = 0;         // classes with keys >= cand: population counts of ballots
 #pragma unroll
             for (int u = 0; u < 4; u++) c += __popcll(lane_mask(key[u] >= cand));
-            if (c >= top_k) kth = cand;
-            if (c == top_k) break;
-        }
+            kth = c >= top_k ? cand : kth;
+            bit >>= 1;
+        } while (c != top_k && bit);
     }
     float w[4], part = 0.0f;
 #pragma unroll
