@@ -29,12 +29,14 @@ from ._lib import YggError, YggInfo, check
 LN2 = math.log(2.0)
 
 
+# (the address as an int, which ctypes converts for a pointer argument: an object less per argument of a step)
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream(device: Optional[int] = None):
+    """The current stream of device (default: the current device) as the pointer the C-ABI takes."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device is None else device)
 
 
 def device_tokens(tokens, vocab: int, device, check_device: bool = False) -> torch.Tensor:
@@ -44,8 +46,11 @@ def device_tokens(tokens, vocab: int, device, check_device: bool = False) -> tor
     read back, which would wait for every launch before them: a kernel stops a stream at a token outside [0, vocab)
     and sets bit 0 of the model's error word (take_errors()). check_device (or YGG_CHECK_TOKENS=1) checks GPU tokens
     too, at the cost of that wait."""
-    if isinstance(tokens, torch.Tensor) and tokens.device.type == "cuda":
-        x = tokens.to(device=device, dtype=torch.int32).contiguous()
+    if isinstance(tokens, torch.Tensor) and tokens.is_cuda:
+        x = tokens
+        if x.dtype != torch.int32 or x.device != device:
+            x = x.to(device=device, dtype=torch.int32)
+        x = x.contiguous()
         if (check_device or os.environ.get("YGG_CHECK_TOKENS") == "1") and x.numel() and \
                 (int(x.min()) < 0 or int(x.max()) >= vocab):
             raise ValueError(f"token out of range [0, {vocab})")
@@ -53,11 +58,15 @@ def device_tokens(tokens, vocab: int, device, check_device: bool = False) -> tor
     a = tokens.numpy() if isinstance(tokens, torch.Tensor) else np.asarray(tokens)
     if a.dtype.kind not in "iu":
         raise ValueError(f"tokens must be integers, got {a.dtype}")
-    if a.size and (a.min() < 0 or a.max() >= vocab):
+    if not a.dtype.isnative:
+        a = a.astype(a.dtype.newbyteorder("="))
+    # (one pass: a negative entry is a large one as unsigned)
+    if a.size and int(a.view(f"u{a.dtype.itemsize}").max()) >= vocab:
         raise ValueError(f"token out of range [0, {vocab})")
-    host = torch.from_numpy(np.ascontiguousarray(a, np.int32))
-    if host.numel():
-        host = host.pin_memory()
+    if not a.size:
+        return torch.empty(a.shape, dtype=torch.int32, device=device)
+    host = torch.empty(a.shape, dtype=torch.int32, pin_memory=True)
+    np.copyto(host.numpy(), a, casting="unsafe")
     return host.to(device, non_blocking=True)
 
 
@@ -91,7 +100,7 @@ class Yggdrasil:
     def __init__(self, path, device=None, graph: bool = False, check_tokens: bool = False):
         if not torch.cuda.is_available():
             raise RuntimeError("backend='hip' needs a ROCm GPU (torch.cuda.is_available() is False)")
-        L = _lib.lib()
+        self._lib = L = _lib.lib()
         self.device = torch.device("cuda", torch.cuda.current_device() if device is None else
                                    torch.device(device).index or 0)
         h = ctypes.c_void_p()
@@ -169,7 +178,7 @@ class Yggdrasil:
         return x
 
     def _check_state(self, state: torch.Tensor, B: int) -> torch.Tensor:
-        if state.dtype != torch.int8 or tuple(state.shape) != (B, self.layers, self.n):
+        if state.dtype != torch.int8 or state.shape != (B, self.layers, self.n):
             raise ValueError(f"state must be int8 {(B, self.layers, self.n)}, got {state.dtype} {tuple(state.shape)}")
         if state.device != self.device:
             raise ValueError(f"state on {state.device}, model on {self.device}")
@@ -180,7 +189,8 @@ class Yggdrasil:
         B = x.shape[0]
         logits = torch.empty(B, self.vocab, dtype=torch.float32, device=self.device)
         out = torch.empty_like(state)
-        check(_lib.lib().ygg_step(self._h, _ptr(x), _ptr(state), _ptr(out), _ptr(logits), None, B, _stream()))
+        check(self._lib.ygg_step(self._h, x.data_ptr(), state.data_ptr(), out.data_ptr(), logits.data_ptr(), None, B,
+                                 _stream()))
         return logits, out
 
     def step(self, tokens, state: torch.Tensor):
@@ -279,23 +289,27 @@ class Yggdrasil:
         windows x against their next tokens y). Rows start from state, or from zero (yggdrasil/inference.py:179-188).
         One fused launch per batch of rows: the step and the float64 log-softmax of the reference's score mode
         (cpu/ygg.cpp:513-516), no logits written."""
-        tokens = np.atleast_2d(np.asarray(tokens, np.int64))
+        def rows_of(a):
+            a = np.asarray(a)
+            return np.atleast_2d(a if a.dtype.kind in "iu" else a.astype(np.int64))
+        tokens = rows_of(tokens)
         if targets is not None:
-            targets = np.atleast_2d(np.asarray(targets, np.int64))
+            targets = rows_of(targets)
             if targets.shape != tokens.shape:
                 raise ValueError(f"targets {targets.shape} for tokens {tokens.shape}")
         out = []
         for i in range(0, len(tokens), batch):
             rows = tokens[i:i + batch]
-            if targets is None:
-                xin, tgt = rows[:, :-1], rows[:, 1:]
-            else:
-                xin, tgt = rows, targets[i:i + batch]
-            B, T = xin.shape
+            B, T = rows.shape[0], rows.shape[1] - (targets is None)
             st = self.init_state(B) if state is None else self._check_state(state[i:i + B], B).clone()
             nll = torch.zeros(B, dtype=torch.float64, device=self.device)
             if T > 0:
-                xd, yd = self._tokens(np.ascontiguousarray(xin)), self._tokens(np.ascontiguousarray(tgt))
+                # (each token is checked and copied once; inputs and targets are parted on the device)
+                xd = self._tokens(rows)
+                if targets is None:
+                    xd, yd = xd[:, :-1].contiguous(), xd[:, 1:].contiguous()
+                else:
+                    yd = self._tokens(targets[i:i + batch])
                 scratch, need = self._scratch(B, T, True)
                 if scratch is not None:
                     check(_lib.lib().ygg_score_scratch(self._h, _ptr(xd), _ptr(yd), B, T, _ptr(st), _ptr(nll),
