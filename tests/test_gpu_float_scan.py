@@ -26,6 +26,7 @@ CASES = [
     (128, 16, 32, 6, 2, 33, 16, True, 2, 130),   # 33 classes: no 16-byte rows
     (256, 33, 64, 4, 2, 40, 256, True, 5, 20),   # the widest rows: 512 router inputs, 3 rank tiles
     (64, 8, 16, 5, 1, 64, 16, True, 6, 40),      # a token layer only
+    (64, 8, 16, 5, 3, 64, 16, True, 40, 420),    # 8400 rows: the route a level a step
 ]
 
 

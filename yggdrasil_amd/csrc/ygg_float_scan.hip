@@ -16,6 +16,7 @@
 // trained shape 3 635 -> 173 us; scoring 256 x 128 of the large one 6 597 -> 939; f64 calibration of 500 x 200 of the
 // medium one 45.6 -> 2.0 ms. The token-by-token kernel is bound by the dependent loads and barriers of a layer (7 us
 // each), this form by its launches (17 to 26 of 4 us) at a thousand rows and by the experts' bytes at tens of thousands.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -136,18 +137,21 @@ template <typename T> __global__ __launch_bounds__(256) void fl_begin(const Floa
 // The route of layer l and its layer input: 16 rows per workgroup, 16 lanes per row. The descent reads one node row per
 // level (rows of a layer stay in L2) with its input row in registers; the product V' rms(h) of the 16 rows is
 // split over the wavefronts by coordinates. EPL: router inputs per lane at most; VW: their vector width (kVE where the
-// token part is whole vectors, else 1).
-template <typename T, int EPL, int VW>
+// token part is whole vectors, else 1). LV: levels a step; two (a node and both its children loaded together, half again
+// the bytes) for few rows, which wait for the loads, one for many. The workgroups' LDS is theirs by n and R2 (route_of),
+// the partial sums where the rows were: a workgroup waits for its loads most of the time, so what counts is how many fit
+// a CU (100k f64 rows of the medium trained shape: 66 KB of LDS and two of them 124 us, 17 KB and eight 83).
+template <typename T, int EPL, int VW, int LV>
 __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const Chunk<T> c, int l) {
-    constexpr int VE = kVE<T>, KC = 4 * VE, LD = kMaxN + VE;
-    __shared__ T f16[16][LD];                 // rms(h_below) of the rows
-    __shared__ T part[4][16][kMaxR2 + 1];
+    constexpr int VE = kVE<T>, KC = 4 * VE, CGS = kMaxR2 / (16 * VE);
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const FloatLayerDev<T> &y = m.layers[l];
-    const int n = m.n, F = m.F, width = F + (m.router_state ? n : 0);
+    const int n = m.n, F = m.F, LD = n + VE, width = F + (m.router_state ? n : 0);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rl = tid & 15, rr = tid >> 4;
     const int row = blockIdx.x * 16 + rr;
     const int s = row / c.Tc;
     const bool live = row < c.N && row - s * c.Tc < c.len(s);
+    T *const f16 = (T *)lds, *const part = (T *)lds;      // rms(h_below) of the rows, LD apart; then [4][16][R2 + 1]
     {
         const T *h = c.h + ((size_t)(l - 1) * c.N + (live ? row : 0)) * n;
         typename Vec<T>::type v[kMaxN / (16 * VE)];
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
             const int e = VE * (rl + 16 * k);
             if (e < n)
 #pragma unroll
-                for (int q = 0; q < VE; q++) f16[rr][e + q] = Vec<T>::at(v[k], q) * rinv;
+                for (int q = 0; q < VE; q++) f16[rr * LD + e + q] = Vec<T>::at(v[k], q) * rinv;
         }
     }
     __syncthreads();
@@ -178,30 +182,57 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
 #pragma unroll
             for (int q = 0; q < VW; q++) {
                 const int e = VW * (rl + 16 * k) + q;
-                f[VW * k + q] = e < F ? emb[e] : (e < width ? f16[rr][e - F] : T(0));
+                f[VW * k + q] = e < F ? emb[e] : (e < width ? f16[rr * LD + e - F] : T(0));
             }
         }
-        int node = 0;
-        for (int d = 0; d < m.D; d++) {
-            const T *w = y.W + (size_t)node * width;
+        // the lane's products with a node's row, loaded by load
+        using Row = std::conditional_t<(VW > 1), typename Vec<T>::type, T>;
+        constexpr int RW = VW > 1 ? EPL / VE : EPL;
+        auto load = [&](Row (&wv)[RW], int at) {
+            const T *w = y.W + (size_t)at * width;
+#pragma unroll
+            for (int k = 0; k < RW; k++) {
+                const int e = VW * (rl + 16 * k);
+                if constexpr (VW > 1) wv[k] = load_vec(w + e, e < width);
+                else wv[k] = load_or_zero(w + e, e < width);
+            }
+        };
+        auto score = [&](const Row (&wv)[RW]) {
             T p = T(0);
-            if constexpr (VW > 1) {
-                typename Vec<T>::type wv[EPL / VE];
 #pragma unroll
-                for (int k = 0; k < EPL / VE; k++) wv[k] = load_vec(w + VE * (rl + 16 * k), VE * (rl + 16 * k) < width);
-#pragma unroll
-                for (int k = 0; k < EPL / VE; k++)
+            for (int k = 0; k < RW; k++) {
+                if constexpr (VW > 1) {
 #pragma unroll
                     for (int q = 0; q < VE; q++) p = fma(f[VE * k + q], Vec<T>::at(wv[k], q), p);
-            } else {
-                T wv[EPL];
-#pragma unroll
-                for (int k = 0; k < EPL; k++) wv[k] = load_or_zero(w + rl + 16 * k, rl + 16 * k < width);
-#pragma unroll
-                for (int k = 0; k < EPL; k++) p = fma(f[k], wv[k], p);
+                } else {
+                    p = fma(f[k], wv[k], p);
+                }
             }
+            return sum16(p);
+        };
+        int node = 0, d = 0;
+        if constexpr (LV == 2) {
+            for (; d + 2 <= m.D; d += 2) {
+                const int at[3] = {node, 2 * node + 1, 2 * node + 2};
+                Row wv[3][RW];
+                T bias[3];
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    load(wv[k], at[k]);
+                    bias[k] = y.bias[at[k]];
+                }
+                T p[3];
+#pragma unroll
+                for (int k = 0; k < 3; k++) p[k] = score(wv[k]) + bias[k];
+                const bool right = p[0] > T(0);
+                node = 2 * (right ? at[2] : at[1]) + 1 + ((right ? p[2] : p[1]) > T(0) ? 1 : 0);
+            }
+        }
+        for (; d < m.D; d++) {
+            Row wv[RW];
+            load(wv, node);
             const T bias = y.bias[node];
-            node = 2 * node + 1 + (sum16(p) + bias > T(0) ? 1 : 0);
+            node = 2 * node + 1 + (score(wv) + bias > T(0) ? 1 : 0);
         }
         if (rl == 0) {
             const int r = node - ((1 << m.D) - 1);
@@ -215,16 +246,18 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
     if (!y.Vd) return;
     const int R2 = m.R2, kk = lane >> 4, cl = lane & 15;
     const bool whole = R2 % VE == 0;
-    for (int c0 = 0; c0 < R2; c0 += 16 * VE) {
-        typename Acc<T>::type acc[VE];
+    typename Acc<T>::type acc[CGS][VE];
 #pragma unroll
-        for (int q = 0; q < VE; q++) acc[q] = typename Acc<T>::type{};
-        const int col = c0 + VE * cl;
+    for (int g = 0; g < CGS; g++) {
+#pragma unroll
+        for (int q = 0; q < VE; q++) acc[g][q] = typename Acc<T>::type{};
+        const int col = 16 * VE * g + VE * cl;
+        if (16 * VE * g >= R2) break;
         for (int j = wave; j < n / KC; j += 4) {
             const int i0 = KC * j + VE * kk;
 #pragma unroll
             for (int u = 0; u < VE; u++) {
-                const T a = f16[cl][i0 + u];
+                const T a = f16[cl * LD + i0 + u];
                 const T *b = y.Vd + (size_t)(i0 + u) * R2 + col;
                 typename Vec<T>::type bv{};
                 if (whole) {
@@ -235,20 +268,30 @@ __global__ __launch_bounds__(256) void fl_route(const FloatDevModel<T> m, const 
                         if (col + q < R2) ((T *)&bv)[q] = b[q];
                 }
 #pragma unroll
-                for (int q = 0; q < VE; q++) acc[q] = mma(a, Vec<T>::at(bv, q), acc[q]);
+                for (int q = 0; q < VE; q++) acc[g][q] = mma(a, Vec<T>::at(bv, q), acc[g][q]);
             }
         }
+    }
+    __syncthreads();      // (every wavefront has read the rows)
+#pragma unroll
+    for (int g = 0; g < CGS; g++) {
+        const int col = 16 * VE * g + VE * cl;
 #pragma unroll
         for (int q = 0; q < VE; q++)
-            if (col + q < kMaxR2)
+            if (col + q < R2)
 #pragma unroll
-                for (int i = 0; i < 4; i++) part[wave][acc_row<T>(i, kk)][col + q] = acc[q][i];
+                for (int i = 0; i < 4; i++)
+                    part[(wave * 16 + acc_row<T>(i, kk)) * (R2 + 1) + col + q] = acc[g][q][i];
     }
     __syncthreads();
     for (int i = tid; i < 16 * c.ZLW; i += 256) {
         const int k = i % c.ZLW, mrow = i / c.ZLW, to = blockIdx.x * 16 + mrow;
         if (to >= c.N) break;
-        const T z = k < R2 ? ((part[0][mrow][k] + part[1][mrow][k]) + part[2][mrow][k]) + part[3][mrow][k] : T(0);
+        T z = T(0);
+        if (k < R2) {
+            auto of = [&](int w) { return part[(w * 16 + mrow) * (R2 + 1) + k]; };
+            z = ((of(0) + of(1)) + of(2)) + of(3);
+        }
         c.zl[((size_t)l * c.N + to) * c.ZLW + k] = z;
     }
 }
@@ -615,10 +658,15 @@ template <typename T> int64_t scratch_of(const FloatDevModel<T> &m, int64_t B, i
     return (int64_t)up256(want < cap ? want : cap);
 }
 
+// Rows below which the route takes two levels a step.
+constexpr int kFewRows = 8192;
+
 template <typename T, int EPL> void route_of(const FloatDevModel<T> &m, const Chunk<T> &c, int l, hipStream_t st) {
-    const dim3 grid((c.N + 15) / 16), wg(256);
-    if (m.F % kVE<T> == 0) hipLaunchKernelGGL((fl_route<T, EPL, kVE<T>>), grid, wg, 0, st, m, c, l);
-    else hipLaunchKernelGGL((fl_route<T, EPL, 1>), grid, wg, 0, st, m, c, l);
+    const size_t rows = 16 * (size_t)(m.n + kVE<T>), parts = 64 * (size_t)(m.R2 + 1), lds = std::max(rows, parts) * sizeof(T);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((c.N + 15) / 16), dim3(256), lds, st, m, c, l); };
+    if (m.F % kVE<T>) go(fl_route<T, EPL, 1, 1>);
+    else if (c.N < kFewRows) go(fl_route<T, EPL, kVE<T>, 2>);
+    else go(fl_route<T, EPL, kVE<T>, 1>);
 }
 
 template <typename T>
@@ -683,12 +731,14 @@ int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T 
                 if (sorted) launch_sort(c.by[l], c.by[0], l == 1, st);
                 const int64_t waves = (int64_t)(sorted ? c.by[l].max_tiles : c.N) * ((m.n + 16 * kVE<T> - 1) / (16 * kVE<T>));
                 const int64_t wgs = (waves + 3) / 4;
-                hipLaunchKernelGGL(fl_input<T>, dim3((unsigned)(wgs < 8192 ? wgs : 8192)), dim3(256), 0, st, m, c, l);
+                // (with the maxima each wavefront ends with additions of its own)
+                const int64_t cap = stats ? 1024 : 8192;
+                hipLaunchKernelGGL(fl_input<T>, dim3((unsigned)(wgs < cap ? wgs : cap)), dim3(256), 0, st, m, c, l);
                 scan(l);
             }
             if (m.L == 1 && sorted) launch_sort(c.by[0], c.by[0], false, st);
             if (logits || stats) {
-                const int64_t wgs = ((int64_t)(sorted ? c.N / kTile + p.E : c.N) + 3) / 4, most = stats ? 1024 : 8192;
+                const int64_t wgs = ((int64_t)(sorted ? c.N / kTile + p.E : c.N) + 3) / 4, most = stats ? 256 : 8192;
                 const dim3 grid((unsigned)(wgs < most ? wgs : most), m.L);
                 auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, m, c); };
                 if (m.R <= 16) stats ? go(fl_readout<T, 1, true>) : go(fl_readout<T, 1, false>);
