@@ -1,0 +1,70 @@
+"""GPU: the f32 step of the trained shapes (float_step in csrc/ygg_float.hip) token by token, against the float64
+restatement oracle/float_oracle.py. A result's sums have at most 288 terms: 288 eps = 3.4e-5 of the terms' size, and the
+decays (at most 1) let it grow over a case's tokens; 2e-4 as for the other f32 forms, before a stream's first route that
+differs."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import float_oracle as FO
+from yggdrasil_amd import _lib
+from yggdrasil_amd import float_model as FM
+
+pytestmark = pytest.mark.gpu
+
+# n, R, R2, depth, layers, vocab, token part, state in the router, streams
+CASES = [
+    (64, 8, 16, 1, 2, 64, 1, True, 3),        # one node; a token part of one
+    (64, 8, 16, 5, 3, 256, 32, True, 5),      # one whole round, the widest token part, 256 classes
+    (64, 8, 16, 6, 3, 33, 16, False, 5),      # two rounds, routing on the token alone
+    (128, 16, 32, 5, 3, 33, 16, False, 4),    # 33 classes
+    (128, 16, 32, 11, 2, 20, 7, True, 4),     # three rounds, the last of one level
+    (256, 32, 64, 4, 5, 20, 32, True, 3),
+    (256, 32, 64, 6, 3, 256, 5, True, 1),
+    (256, 32, 64, 4, 2, 20, 33, True, 3),     # a token part of 33: the general build
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
+def test_step_equals_restatement(case):
+    import torch
+    n, R, R2, D, L, V, F, rs, B = case
+    print(f"case {case}", flush=True)
+    spec = FM.FloatSpec(d_state=n, block_size=16, router_depth=D, vocab=V, n_layers=L, router_token_dim=F,
+                        input_rank=8, readout_rank=R, layer_input_rank=R2, router_state=rs)
+    raw, ob = FM.from_params(FM.random_params(spec, 5))
+    layers = FM.float_layers(raw)
+    T = 24
+    x = np.random.default_rng(4).integers(0, V, (B, T))
+    first = FO.run(layers, ob, x[:, :4])
+    ref = FO.run(layers, ob, x[:, 4:], state=first["state"])
+    m, lib = FM.FloatYggdrasil(layers, ob, precision=32), _lib.lib()
+    assert m.kernel_name == ("ygg::float_kernel<float>" if F > 32 else
+                             "ygg::float_kernel<float, %d, %d, %d, 16>" % (n, R, R2)), m.kernel_name
+    end = T - 4 if B == 1 else 9                # the last stream ends at a token outside [0, V)
+    if B > 1:
+        x[-1, 4 + end] = V
+    st = torch.tensor(first["state"], dtype=m.dtype, device=m.device)
+    xd = torch.tensor(x[:, 4:], dtype=torch.int32, device=m.device).contiguous()
+    lg = torch.full((B, T - 4, V), 7.0, dtype=m.dtype, device=m.device)
+    lv = torch.full((B, T - 4, L), -5, dtype=torch.int32, device=m.device)
+    p = [ctypes.c_void_p(t.data_ptr()) for t in (xd, st, lg, lv)]
+    q = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib.ygg_float_run(m._h, p[0], B, T - 4, p[1], p[2], p[3], None, q))
+    e = ctypes.c_uint32()
+    _lib.check(lib.ygg_float_take_errors(m._h, q, ctypes.byref(e)))
+    assert e.value == (1 if B > 1 else 0)
+    lg, lv, st = lg.cpu().numpy(), lv.cpu().numpy(), st.cpu().numpy()
+    split = 0
+    for s in range(B):
+        t1 = end if s == B - 1 else T - 4
+        d = (lv[s, :t1] != ref["leaves"][s, :t1]).any(-1)
+        upto = int(np.argmax(d)) if d.any() else t1
+        split += upto < t1
+        np.testing.assert_allclose(lg[s, :upto], ref["logits"][s, :upto], rtol=2e-4, atol=2e-4)
+        assert (lg[s, t1:] == 7.0).all() and (lv[s, t1:] == -5).all()
+        if upto == t1 == T - 4:
+            np.testing.assert_allclose(st[s], ref["state"][s], rtol=2e-4, atol=2e-4)
+    assert split <= 1
+    m.close()

@@ -12,9 +12,7 @@
 // the round's subtree (every load of a round issued at once, the input row held in registers for the layer); for the
 // layer input wavefront q sums its quarter of the coordinates for row k = lane of V'; thread i owns coordinate i of
 // the update (its table entry, U' column and A row loaded together); the readout takes 256 / R threads per row of P;
-// thread c owns class c of the logits. The builds specialised on a shape issue a layer's constant loads (Q's column
-// of each class, V''s share of each thread) at the layer's start, before its route, and the readout's P row with the
-// update's record, so that a layer waits for the route's rounds and one record load only.
+// thread c owns class c of the logits. The reference's trained shapes have f32 builds of their own (float_step).
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -23,6 +21,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "ygg_float.h"
@@ -75,16 +74,217 @@ template <typename T> __device__ __forceinline__ T block_sum(T v, T *red, int ti
 constexpr int kRouteGroup = 16;                           // threads per node of a router round
 constexpr int kRouteElems = (kMaxF + kMaxN) / kRouteGroup; // router inputs per thread at most
 
+// The f32 step of the reference's trained shapes: 4 N threads per stream (its 1024 threads at n = 256 are a CU's), so that
+// a layer's loads are many threads' and short. Per layer, for G = 32 lanes a node at n = 256, 16 at 128, 8 at 64:
+//   route    rounds of 5 levels, the 31 nodes of a subtree on G lanes each; a round's decisions are bits of one LDS word
+//   V' h     thread (k, part): row k over a sixteenth of the coordinates; the parts are summed after the first round
+//   update   thread (i, quarter): a quarter of coordinate i's U' and A terms; the quarters are summed by thread i
+//   readout  32 lanes per row of P; logits: thread (class, part) 8 ranks of the class, its parts summed once per token
+// The next layer's V', first round and token part are loaded behind the current one's update, so a layer waits for two
+// dependent loads, its second round and its expert's record, and meets five barriers: latency bounds it until the streams
+// fill the chip. Depth 10, 5 layers, 4 tokens of 1 / 16 / 256 / 1024 streams (us; before, on 256 threads with three rounds
+// of 4 levels and 13 barriers a layer): n = 64 54 / 55 / 58 / 71 (132 / 134 / 135 / 531), n = 128 57 / 58 / 76 / 152
+// (148 / 151 / 161 / 629), n = 256 87 / 93 / 121 / 455 (189 / 193 / 219 / 837).
+template <int G> __device__ __forceinline__ float lanes_sum(float v) {
+    auto move = [&](auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v += move(std::integral_constant<int, 0xB1>());      // quad_perm 1 0 3 2
+    v += move(std::integral_constant<int, 0x4E>());      // quad_perm 2 3 0 1
+    if constexpr (G >= 8) v += move(std::integral_constant<int, 0x141>());     // row_half_mirror
+    if constexpr (G >= 16) v += move(std::integral_constant<int, 0x140>());    // row_mirror
+    if constexpr (G >= 32) v += __shfl_xor(v, 16);
+    return v;
+}
+
+// base[i], its offset in 32 bits beside a uniform base (a 64-bit address per thread and array does not fit the registers)
+__device__ __forceinline__ const float *from(const float *base, uint32_t i) {
+    return (const float *)((const char *)base + i * 4u);
+}
+
+template <int N, int R, int R2>
+__device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const int32_t *__restrict__ tokens, int Tn,
+                                           float *__restrict__ state, float *__restrict__ logits,
+                                           int32_t *__restrict__ leaves) {
+    constexpr int NT = 4 * N, G = N / 8, PARTS = NT / R2, VC = N / PARTS, UK = R2 / 4,
+                  PL = 32, PE = N / PL, FE = kStepF / G, QP = NT / 256, RQ = R / QP;
+    static_assert(NT / R == PL && PARTS == 16 && RQ == 8, "the trained shapes' proportions");
+    __shared__ float hs[YGG_MAX_LAYERS][N];   // states
+    __shared__ float bl[N], hn[N];            // rms(h) of the layer below; the new state
+    __shared__ float zp[PARTS][R2 + 1], zl[R2], up[4][N], zs[R], red[N / 64], lgp[QP][256];
+    __shared__ uint32_t dec[4];               // a round's decisions, a bit per node of its subtree
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, L = m.L, V = m.V, C = m.classes, F = m.F, D = m.D;
+    const bool rs = m.router_state != 0;
+    float *st = state + (size_t)s * L * N;
+    for (int i = tid; i < L * N; i += NT) hs[i / N][i % N] = st[i];
+    if (tid < 4) dec[tid] = 0u;
+    __syncthreads();
+    const int32_t *tok = tokens + (size_t)s * Tn;
+    for (int t = 0; t < Tn; t++) {
+        const int x = __builtin_amdgcn_readfirstlane(tok[t]);
+        if (x < 0 || x >= V) {
+            if (tid == 0) atomicOr(m.err, 1u);
+            break;
+        }
+        float lg = 0.0f, vv[VC], w[N / G], wt[FE], emb[FE], bias = 0.0f;
+        int rg = 0, rl = 0, vk = 0, vp = 0, ui = 0, uq = 0, qc = 0, qp = 0, kdep = 0, path = 0;
+        // this thread's places, computed again in each layer (hidden from the compiler: every array's offset kept over
+        // the loop does not fit the registers at n = 256, 26 of them spilled)
+        auto places = [&] {
+            int i = tid;
+            asm volatile("" : "+v"(i));
+            i &= NT - 1;
+            rg = i / G, rl = i % G, vk = i % R2, vp = i / R2, ui = i % N, uq = i / N, qc = i & 255, qp = i >> 8;
+            kdep = 31 - __builtin_clz(rg + 1), path = rg + 1 - (1 << kdep);     // node rg of a subtree
+        };
+        // layer l's V', token part and the rows of its round from node `root` (heap order) of h levels
+        auto load_below = [&](int l) {
+            const float *v = from(m.layers[l].Vd, vp * VC * R2 + vk);
+#pragma unroll
+            for (int i = 0; i < VC; i++) vv[i] = v[i * R2];
+            const float *e = m.layers[l].emb + (size_t)x * F;
+#pragma unroll
+            for (int k = 0; k < FE; k++) emb[k] = *from(e, min(rl + G * k, F - 1));
+        };
+        auto load_round = [&](int l, int root, int h) {
+            const int node = ((root + 1) << kdep) - 1 + path;
+            const int at = rg < (1 << h) - 1 ? node : 0;      // (lanes past the round's nodes: a row that nobody reads)
+            const uint32_t row = (uint32_t)at * (F + (rs ? N : 0));      // (at most 2^20 rows of 288)
+#pragma unroll
+            for (int k = 0; k < FE; k++) wt[k] = *from(m.layers[l].W, row + min(rl + G * k, F - 1));
+            const float *ws = rs ? from(m.layers[l].W, row + F + rl) : from(m.layers[l].P, rl);   // (P: not used)
+#pragma unroll
+            for (int k = 0; k < N / G; k++) w[k] = ws[G * k];
+            bias = *from(m.layers[l].bias, at);
+        };
+        for (int l = 0; l < L; l++) {
+            const FloatLayerDev<float> &y = m.layers[l];
+            int r = x;
+            places();
+            // 8 ranks of class qc's column of Q^T
+            float qw[RQ];
+#pragma unroll
+            for (int j = 0; j < RQ; j++) qw[j] = *from(y.Q + j * C, qp * RQ * C + min(qc, C - 1));
+            if (l > 0) {
+                float f[N / G];
+#pragma unroll
+                for (int k = 0; k < N / G; k++) f[k] = bl[rl + G * k];
+                float z = 0.0f;
+#pragma unroll
+                for (int i = 0; i < VC; i++) z = fmaf(vv[i], bl[vp * VC + i], z);
+                zp[vp][vk] = z;
+                int root = 0;
+                for (int d0 = 0, rd = 0; d0 < D; d0 += 5, rd++) {
+                    const int h = D - d0 < 5 ? D - d0 : 5;
+                    if (rd) load_round(l, root, h);
+                    float p = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < FE; k++) p = rl + G * k < F ? fmaf(emb[k], wt[k], p) : p;
+                    if (rs) {
+#pragma unroll
+                        for (int k = 0; k < N / G; k++) p = fmaf(f[k], w[k], p);
+                    }
+                    p = lanes_sum<G>(p);
+                    if (rl == 0 && rg < (1 << h) - 1 && p + bias > 0.0f) atomicOr(&dec[rd], 1u << rg);
+                    __syncthreads();
+                    if (rd == 0 && tid < R2) {
+                        float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int q = 0; q < PARTS; q++) a[q % 4] += zp[q][tid];
+                        zl[tid] = (a[0] + a[1]) + (a[2] + a[3]);
+                    }
+                    const uint32_t bits = dec[rd];
+                    int j = 0;
+                    for (int k = 0; k < h; k++) j = 2 * j + 1 + ((bits >> j) & 1u);
+                    root = ((root + 1) << h) - 1 + (j - ((1 << h) - 1));
+                }
+                r = __builtin_amdgcn_readfirstlane(root - ((1 << D) - 1));
+                if (D <= 5) __syncthreads();        // (zl, where no second round's barrier follows it)
+            }
+            // the expert's record: this thread's share of U', A and P; then the next layer's loads behind it
+            float uw[UK], pw[PE], tab = 0.0f;
+            if (l > 0) {
+                const float *u = from(y.Up + (size_t)r * R2 * N, uq * UK * N + ui);
+#pragma unroll
+                for (int k = 0; k < UK; k++) uw[k] = u[k * N];
+            }
+            const float4 aw = *(const float4 *)from(y.A + (size_t)r * N * 16, (ui / 16) * 256 + a_index<float>(16, ui % 16, 4 * uq));
+            if (uq == 0) tab = *from(y.table + (l == 0 ? (size_t)x : (size_t)r * V + x) * N, ui);
+            const int prow = (uq * N + ui) / PL, pu = ui % PL;
+            const float *pr = from(y.P + (size_t)r * R * N, prow * N + pu);
+#pragma unroll
+            for (int e = 0; e < PE; e++) pw[e] = pr[PL * e];
+            if (l + 1 < L) {
+                load_below(l + 1);
+                load_round(l + 1, 0, D < 5 ? D : 5);
+            }
+            float a = 0.0f, b = 0.0f;
+            if (l > 0) {
+#pragma unroll
+                for (int k = 0; k < UK; k++) a = fmaf(uw[k], zl[uq * UK + k], a);
+            }
+            const float *ho = hs[l] + (ui & ~15) + 4 * uq;
+            b = fmaf(aw.x, ho[0], b);
+            b = fmaf(aw.y, ho[1], b);
+            b = fmaf(aw.z, ho[2], b);
+            b = fmaf(aw.w, ho[3], b);
+            up[uq][ui] = a + b;
+            __syncthreads();
+            if (tid < N) {
+                const float h = tab + ((up[0][ui] + up[1][ui]) + (up[2][ui] + up[3][ui]));
+                hn[ui] = h;
+                hs[l][ui] = h;
+                const float ss = wave_sum(h * h);
+                if (lane == 0) red[tid >> 6] = ss;
+            }
+            if (tid < 4) dec[tid] = 0u;
+            __syncthreads();
+            float ss = 0.0f;
+#pragma unroll
+            for (int k = 0; k < N / 64; k++) ss += red[k];
+            if (tid < N) bl[ui] = hn[ui] * (1.0f / sqrtf(ss / (float)N + (float)kRmsEps));
+            float z = 0.0f;
+#pragma unroll
+            for (int e = 0; e < PE; e++) z = fmaf(pw[e], hn[pu + PL * e], z);
+            z = lanes_sum<PL>(z);
+            if (pu == 0) zs[prow] = z;
+            __syncthreads();
+            float q = 0.0f;
+#pragma unroll
+            for (int j = 0; j < RQ; j++) q = fmaf(qw[j], zs[qp * RQ + j], q);
+            lg += q;
+            if (leaves && tid == 0) leaves[((size_t)s * Tn + t) * L + l] = r;
+        }
+        if (logits) {
+            lgp[qp][qc] = lg;
+            __syncthreads();
+            if (tid < C) {
+                float v = lgp[0][tid];
+#pragma unroll
+                for (int k = 1; k < QP; k++) v += lgp[k][tid];
+                logits[((size_t)s * Tn + t) * C + tid] = m.output_bias[tid] + v;
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < L * N; i += NT) st[i] = hs[i / N][i % N];
+}
+
 // stats (calibration maxima, cpu/export.py:127-153), per layer: [|h|, |V' rms(h_below)|, |P_r h|, |h| per 16
 // coordinates (n/16), |P_r h| per row (R)]
-// NS, RS, R2S, BS: the state width, readout rank, layer-input rank and block size at compile time (the reference's
-// trained shapes: every row length a constant), or 0 for the model's (any shape the loader takes)
+// NS, RS, R2S, BS: the state width, readout rank, layer-input rank and block size of a float_step build (the reference's
+// trained shapes; no stats), or 0 for the model's (any shape the loader takes)
 // (one wavefront per SIMD: the unrolled row loads of a thread are its registers)
 template <typename T, int NS = 0, int RS = 0, int R2S = 0, int BS = 0>
-__global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void float_kernel(
+__global__ __launch_bounds__(NS ? 4 * NS : kFThreads)
+__attribute__((amdgpu_waves_per_eu(NS ? NS / 64 : 1, NS ? 8 : 1))) void float_kernel(
     const FloatDevModel<T> m, const int32_t *__restrict__ tokens, int Tn, T *__restrict__ state,
     T *__restrict__ logits, int32_t *__restrict__ leaves, double *__restrict__ stats) {
-    constexpr int MN = NS ? NS : kMaxN, MR = RS ? RS : kMaxR, MR2 = R2S ? R2S : kMaxR2, MB = BS ? BS : kMaxB;
+    if constexpr (NS != 0) {
+        float_step<NS, RS, R2S>(m, tokens, Tn, state, logits, leaves);
+        return;
+    } else {
+    constexpr int MN = kMaxN, MR = kMaxR, MR2 = kMaxR2, MB = kMaxB;
     __shared__ T hs[YGG_MAX_LAYERS][kMaxN];   // states
     __shared__ T bl[kMaxN];                   // rms(h) of the layer below
     __shared__ T hn[kMaxN];                   // the new state of the current layer
@@ -95,12 +295,9 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
     __shared__ int dec[16];                   // a router round's decisions, by breadth-first node of its subtree
     __shared__ double gmax[YGG_MAX_LAYERS][kMaxN / 16];
 
-    // PF (the specialised builds): a layer's loads issued early (see above); the general builds load at each use
-    constexpr bool PF = NS != 0;
-    constexpr int PE = RS ? (NS * RS + kFThreads - 1) / kFThreads : MN / 4;   // readout coordinates per thread
+    constexpr int PE = MN / 4;   // readout coordinates per thread
     const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-    const int L = m.L, n = NS ? NS : m.n, b = BS ? BS : m.b, V = m.V, C = m.classes, R = RS ? RS : m.R,
-              R2 = R2S ? R2S : m.R2, F = m.F;
+    const int L = m.L, n = m.n, b = m.b, V = m.V, C = m.classes, R = m.R, R2 = m.R2, F = m.F;
     const int width = F + (m.router_state ? n : 0);
     // readout: TPR threads per row of P (a power of 2 of at most 64 lanes), its coordinates u, u + TPR, ...
     int Rp = 1;
@@ -153,10 +350,6 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                     for (int i = 0; i < MN / 4; i++) vv[i] = i < vlen ? vc[(size_t)i * R2] : T(0);
                 }
             };
-            if constexpr (PF) {
-                load_q();
-                load_v();
-            }
             if (l > 0) {
                 // router descent over f = [router_embed[x]; rms(h_below)], in rounds of up to 4 levels
                 T f[kRouteElems];
@@ -197,7 +390,7 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                 // the layer input zl = V' rms(h_below): each wave's partial sum for row k = lane over its quarter of
                 // the coordinates, the four partials then added in quarter order
                 if (y.Vd) {
-                    if constexpr (!PF) load_v();
+                    load_v();
                     if (vlive) {
                         T a = T(0);
 #pragma unroll
@@ -250,7 +443,6 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                     for (int j = 0; j < MB; j++) aw[j] = (ta && j < b) ? ablk[a_index<T>(b, ii, j)] : T(0);
                 }
                 T h = trow[i];
-                if constexpr (PF) load_p();
                 if (up) {
                     T a = T(0);
 #pragma unroll
@@ -267,8 +459,6 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                 }
                 hv = h;
                 if (stats) smax[l] = fmax(smax[l], (double)fabs(h));
-            } else if constexpr (PF) {
-                load_p();
             }
             // (every thread has read hs[l] before it is overwritten below)
             const T ss = block_sum(tid < n ? hv * hv : T(0), red, tid);
@@ -285,7 +475,7 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
             if (tid < n) bl[tid] = hv * rinv;
             __syncthreads();
             // z = P_r h (every load issued at once)
-            if constexpr (!PF) load_p();
+            load_p();
             if (prow < R) {
                 T a = T(0);
 #pragma unroll
@@ -299,7 +489,7 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
             }
             __syncthreads();
             // logits += Q z, thread c for class c
-            if constexpr (!PF) load_q();
+            load_q();
             if (tid < C) {
                 T a = T(0);
 #pragma unroll
@@ -327,6 +517,7 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(1, 1)
                 atomic_max_nonneg(&stats[(size_t)l * sstride + 3 + g], gmax[l][g]);
             if (prow < R && pu == 0) atomic_max_nonneg(&stats[(size_t)l * sstride + 3 + n / 16 + prow], zmax[l]);
         }
+    }
     }
 }
 
@@ -473,14 +664,15 @@ int ygg_float_run(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, vo
     if (m->precision == 32) {
         // the reference's trained shapes (configs/*/{small,medium,large}.yaml: block 16) have builds of their own
         const FloatDevModel<float> &fm = m->m32;
-        auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3(B), dim3(kFThreads), 0, (hipStream_t)stream, fm, d_tokens, T,
+        auto go = [&](auto kernel, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(B), dim3(threads), 0, (hipStream_t)stream, fm, d_tokens, T,
                                (float *)d_state, (float *)d_logits, d_leaves, d_stats);
         };
-        if (fm.b == 16 && fm.n == 64 && fm.R == 8 && fm.R2 == 16) go(float_kernel<float, 64, 8, 16, 16>);
-        else if (fm.b == 16 && fm.n == 128 && fm.R == 16 && fm.R2 == 32) go(float_kernel<float, 128, 16, 32, 16>);
-        else if (fm.b == 16 && fm.n == 256 && fm.R == 32 && fm.R2 == 64) go(float_kernel<float, 256, 32, 64, 16>);
-        else go(float_kernel<float>);
+        const bool step = float_steps(fm) && !d_stats;
+        if (step && fm.n == 64) go(float_kernel<float, 64, 8, 16, 16>, 256);
+        else if (step && fm.n == 128) go(float_kernel<float, 128, 16, 32, 16>, 512);
+        else if (step && fm.n == 256) go(float_kernel<float, 256, 32, 64, 16>, 1024);
+        else go(float_kernel<float>, kFThreads);
     } else
         hipLaunchKernelGGL(float_kernel<double>, dim3(B), dim3(kFThreads), 0, (hipStream_t)stream, m->m64, d_tokens, T,
                            (double *)d_state, (double *)d_logits, d_leaves, d_stats);
