@@ -621,33 +621,53 @@ __global__ __launch_bounds__(256) void fl_logits(const FloatDevModel<T> m, const
 }
 
 // ------------------------------------------------------------------------------------------------------ host side
-// Sorting pays once an expert has about two rows on average (the sort's launches against reading experts again)
-bool sort_pays(int64_t N, int E) { return E <= kSortLeaves && N >= 2 * (int64_t)E; }
+// Bytes of an expert's record (A, U' and P) a row reads
+template <typename T> int64_t record_bytes(const FloatDevModel<T> &m) { return (int64_t)sizeof(T) * m.n * (16 + m.R2 + m.R); }
+
+// Sorting pays once it keeps about 130 MB of experts' records from being read again: its launches cost 60 to 80 us. Rows
+// where both are as fast, 1024 experts, depth 10 (n = 64 / 128 / 256): f32 about 14000 / 5000 / 2000, f64 6500 / 2500 /
+// 1200, which is 130 to 160, 160 and 230 to 270 MB; 8192 rows in f32, sorted / not: 247 / 218, 283 / 321, 438 / 778 us.
+constexpr int64_t kSortBytes = 130'000'000;
+bool sort_pays(int64_t N, int E, int64_t record) { return E <= kSortLeaves && N > E && (N - E) * record >= kSortBytes; }
 
 struct Plan {
     int64_t fixed, per_row;      // workspace bytes besides the rows' and per row (arrays rounded up apart)
     int E, ZLW, ZW;
+    int64_t record;              // bytes of an expert's record
 };
 
 template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
     Plan p{};
     const int64_t leaves = m.L > 1 ? (int64_t)1 << m.D : 1;
     p.E = (int)(leaves > m.V ? leaves : m.V);
+    p.record = record_bytes(m);
     p.ZLW = (m.R2 + 15) / 16 * 16;
     p.ZW = (m.L * m.R + 15) / 16 * 16;
     p.per_row = (int64_t)sizeof(T) * ((int64_t)m.L * (m.n + p.ZLW) + p.ZW) + 4 + m.L * kSortRowBytes;
-    p.fixed = 256 * 8 + B * 4 + kPad * (4 + (int64_t)m.n * sizeof(T)) + m.L * sort_fixed_bytes(B * Tn, p.E, sort_pays(B * Tn, p.E));
+    p.fixed = 256 * 8 + B * 4 + kPad * (4 + (int64_t)m.n * sizeof(T)) +
+              m.L * sort_fixed_bytes(B * Tn, p.E, sort_pays(B * Tn, p.E, p.record));
     return p;
 }
 
-// Calls of fewer than 4 tokens stay on the step kernel, and so do transition blocks other than 16. At 4 tokens of 1 / 16 /
-// 256 / 1024 streams (us, step kernel / this form): small 132/77, 134/84, 135/98, 531/177; medium 148/90, 151/95, 161/127,
-// 629/214; large 189/113, 193/148, 219/227, 837/387; at fewer tokens the launches cost more than they save.
+// Calls of fewer than 4 tokens stay on the step kernel, and so do transition blocks other than 16. A model without a
+// step build of its own comes here from 4 tokens: the general step took, at 4 tokens of 1 / 16 / 256 / 1024 streams (us,
+// step / this form), small 132/77, 134/84, 135/98, 531/177; medium 148/90, 151/95, 161/127, 629/214; large 189/113,
+// 193/148, 219/227, 837/387. With one (float_steps) the cheaper is estimated: a step's tokens, by rounds of the streams
+// that fit the chip, against this form's launches, the records its rows read (1.2 TB/s) and the sort. Measured at 4 and 8
+// tokens: small, 1 stream 54/75 104/77, 256 58/96 112/105, 1024 71/150 139/169; medium 57/90 109/91, 76/125 146/146,
+// 152/190 295/248; large 87/115 182/117, 121/230 230/326, 455/388 892/435.
 constexpr int kScanTokens = 4;
 constexpr int64_t kScratchCap = (int64_t)1 << 30;
 
 template <typename T> bool takes(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
-    return m.b == 16 && B > 0 && Tn >= kScanTokens;
+    if (m.b != 16 || B <= 0 || Tn < kScanTokens) return false;
+    if (!float_steps(m)) return true;
+    const int64_t N = B * Tn, leaves = m.L > 1 ? (int64_t)1 << m.D : 1, E = leaves > m.V ? leaves : m.V;
+    const bool sorted = sort_pays(N, (int)E, record_bytes(m));
+    const double step = (double)Tn * ((B * m.n + 65535) / 65536) * (12.5 + m.n * m.n / 4096.0);
+    const double scan = 60 + m.n / 4.0 + (double)(sorted ? E : N) * record_bytes(m) * 8.3e-7 +
+                        (sorted ? 60 + (double)N * m.n * sizeof(T) * 1.8e-5 : 0.0);
+    return scan < step;
 }
 
 template <typename T> int64_t scratch_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
@@ -696,7 +716,7 @@ int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T 
             c.N = c.Bc * c.Tc;
             c.ZLW = p.ZLW;
             c.ZW = p.ZW;
-            const bool sorted = sort_pays(c.N, p.E);
+            const bool sorted = sort_pays(c.N, p.E, p.record);
             c.state = state;
             c.logits = logits;
             c.leaves = leaves;
