@@ -238,6 +238,11 @@ int64_t ygg_float_scratch(const ygg_fmodel *m, int B, int T);
 int ygg_float_run_scratch(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, void *d_state, void *d_logits,
                           int32_t *d_leaves, double *d_stats, void *d_scratch, int64_t scratch_bytes, void *stream);
 
+/* The f64 nats -log softmax(logits[i])[next[i]] of `rows` rows of the float model's logits (its precision, [rows][classes],
+   as ygg_float_run leaves them); NaN where next[i] is no class. */
+int ygg_float_nll(const ygg_fmodel *m, const void *d_logits, const int32_t *d_next, int64_t rows, double *d_nll,
+                  void *stream);
+
 /* Wait for `stream`, then return and clear the float model's error word (bit 0: a token outside [0, vocab)). */
 int ygg_float_take_errors(const ygg_fmodel *m, void *stream, uint32_t *errors);
 

@@ -26,6 +26,41 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("classes,rows", [(1, 3), (27, 17), (64, 16), (65, 1), (256, 33)])
+def test_nll_equals_log_softmax(classes, rows, precision):
+    """ygg_float_nll against log-sum-exp in f64: the logits are exact in both, so a sum of at most 256 exponentials of
+    about an ulp each and its logarithm: 1e-13 of values of at most about 200. Ends of the types, a row of one infinity
+    and rows without a class (NaN)."""
+    import torch
+    spec = FM.FloatSpec(d_state=16, block_size=16, router_depth=2, vocab=classes, n_layers=1, router_token_dim=4,
+                        input_rank=4, readout_rank=4, layer_input_rank=0)
+    raw, ob = FM.from_params(FM.random_params(spec, 3))
+    m = FM.FloatYggdrasil(FM.float_layers(raw), ob, precision=precision)
+    rng = np.random.default_rng(classes)
+    lg = (rng.normal(size=(rows, classes)) * 30).astype(np.float32 if precision == 32 else np.float64)
+    lg[0, 0] = -np.inf if classes > 1 else 1.0
+    if rows > 2:
+        lg[1] += np.float32(3e38) if precision == 32 else 1e300
+        lg[2, -1] = np.finfo(lg.dtype).min
+    y = rng.integers(0, classes, rows).astype(np.int32)
+    y[0] = classes - 1
+    if rows > 3:
+        y[3], y[4] = classes, -1
+    wide = lg.astype(np.float64)
+    top = wide.max(-1)
+    ok = (y >= 0) & (y < classes)
+    ref = np.log(np.exp(wide - top[:, None]).sum(-1)) - (wide[np.arange(rows), np.where(ok, y, 0)] - top)
+    a, b = torch.tensor(lg, device=m.device), torch.tensor(y, device=m.device)
+    r = torch.full((rows,), 9.0, dtype=torch.float64, device=m.device)
+    _lib.check(_lib.lib().ygg_float_nll(m._h, a.data_ptr(), b.data_ptr(), rows, r.data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream))
+    r = r.cpu().numpy()
+    assert np.isnan(r[~ok]).all()
+    np.testing.assert_allclose(r[ok], ref[ok], rtol=1e-13, atol=1e-13)
+    m.close()
+
+
 @pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
 def test_step_equals_restatement(case):
     import torch

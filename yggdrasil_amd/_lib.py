@@ -18,7 +18,7 @@ SYMBOLS = ("ygg_load", "ygg_load_blob", "ygg_model_info", "ygg_free", "ygg_step"
            "ygg_run_grouped_noalloc", "ygg_softmax", "ygg_score", "ygg_scratch", "ygg_run_scratch",
            "ygg_score_scratch",
            "ygg_generate", "ygg_take_errors", "ygg_float_load", "ygg_float_run", "ygg_float_scratch",
-           "ygg_float_run_scratch", "ygg_float_take_errors",
+           "ygg_float_run_scratch", "ygg_float_nll", "ygg_float_take_errors",
            "ygg_float_free", "ygg_kernel_name", "ygg_spec_stats", "ygg_last_error", "ygg_version")
 
 ERRORS = {1: "io", 2: "format", 3: "limits", 4: "nomem", 5: "arg", 6: "token", 7: "device"}
@@ -92,6 +92,7 @@ def lib() -> ctypes.CDLL:
     L.ygg_float_scratch.argtypes = [vp, i32, i32]
     L.ygg_float_scratch.restype = ctypes.c_int64
     L.ygg_float_run_scratch.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp, ctypes.c_int64, vp]
+    L.ygg_float_nll.argtypes = [vp, vp, vp, ctypes.c_int64, vp, vp]
     L.ygg_float_take_errors.argtypes = [vp, vp, ctypes.POINTER(ctypes.c_uint32)]
     L.ygg_float_free.argtypes = [vp]
     L.ygg_float_free.restype = None

@@ -339,15 +339,17 @@ class FloatYggdrasil:
     def score(self, tokens, state=None, batch: int = 1024) -> np.ndarray:
         """Bits of tokens[:, 1:] given the tokens before them, per row of tokens (B, L), float64 (B,)."""
         import torch
+        from .inference import device_tokens
         tokens = np.atleast_2d(np.asarray(tokens, np.int64))
         out = []
         for i in range(0, len(tokens), batch):
             x = tokens[i:i + batch]
             st = None if state is None else state[i:i + len(x)]
-            lg = self.run(x[:, :-1], st)["logits"].double()
-            y = torch.as_tensor(x[:, 1:], device=self.device)
-            nll = -torch.log_softmax(lg, -1).gather(-1, y[..., None])[..., 0].sum(-1)
-            out.append((nll / LN2).cpu().numpy())
+            lg = self.run(x[:, :-1], st)["logits"]
+            y = device_tokens(x[:, 1:], self.classes, self.device)
+            nll = torch.empty(y.shape, dtype=torch.float64, device=self.device)
+            check(_lib.lib().ygg_float_nll(self._h, _ptr(lg), _ptr(y), y.numel(), _ptr(nll), _stream()))
+            out.append((nll.sum(-1) / LN2).cpu().numpy())
         return np.concatenate(out) if out else np.zeros(0)
 
     def generate(self, prompt, n: int, temperature: float = 1.0, top_k: int = 0, seed: int = 0):
