@@ -13,8 +13,8 @@
 // the layers' ranks). The rows of few tokens are not sorted (a tile is one row then).
 //
 // Measured against the token-by-token kernel (whole calls, f32 unless said): 9 streams x 100 tokens of the medium
-// trained shape 3 635 -> 173 us; scoring 256 x 128 of the large one 6 597 -> 939; f64 calibration of 500 x 200 of the
-// medium one 45.6 -> 2.0 ms. The token-by-token kernel is bound by the dependent loads and barriers of a layer (7 us
+// trained shape 3 635 -> 169 us; scoring 256 x 128 of the large one 6 597 -> 884; f64 calibration of 500 x 200 of the
+// medium one 45.6 -> 1.63 ms. The general step kernel is bound by the dependent loads and barriers of a layer (7 us
 // each), this form by its launches (17 to 26 of 4 us) at a thousand rows and by the experts' bytes at tens of thousands.
 #include <algorithm>
 #include <cstdlib>

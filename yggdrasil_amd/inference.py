@@ -136,8 +136,9 @@ class Yggdrasil:
         return cls(path, **kw)
 
     def kernel_name(self, B: int, T: int, generate: bool = False, score: bool = False) -> str:
-        """The kernel a call of B streams and T tokens launches (generate: `generate` of T tokens; score: `score`, or
-        `run` with a digest), by the name profilers show for it."""
+        """The kernel a call of B streams and T tokens launches token by token (generate: `generate` of T tokens; score:
+        `score`, or `run` with a digest), by the name profilers show for it; calls of known tokens that go layer by layer
+        (ygg_scratch > 0) launch the kernels of csrc/ygg_scan.hip."""
         if generate and score:
             raise ValueError("generate and score are different calls")
         buf = ctypes.create_string_buffer(128)
