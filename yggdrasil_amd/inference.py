@@ -39,6 +39,25 @@ def _stream(device: Optional[int] = None):
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device is None else device)
 
 
+def host_tokens(tokens, vocab: int) -> np.ndarray:
+    """tokens given on the host as an integer array of the machine's byte order, all of them in [0, vocab) (ValueError)."""
+    a = tokens.numpy() if isinstance(tokens, torch.Tensor) else np.asarray(tokens)
+    if a.dtype.kind not in "iu":
+        raise ValueError(f"tokens must be integers, got {a.dtype}")
+    if not a.dtype.isnative:
+        a = a.astype(a.dtype.newbyteorder("="))
+    if a.size:
+        # one pass: as unsigned, a negative entry is at least half the type's range. A vocabulary past that half (int8:
+        # 129 and more) holds every entry that is not negative.
+        if a.dtype.kind == "i" and vocab > 1 << (8 * a.dtype.itemsize - 1):
+            bad = int(a.min()) < 0
+        else:
+            bad = int(a.view(f"u{a.dtype.itemsize}").max()) >= vocab
+        if bad:
+            raise ValueError(f"token out of range [0, {vocab})")
+    return a
+
+
 def device_tokens(tokens, vocab: int, device, check_device: bool = False) -> torch.Tensor:
     """tokens as a contiguous int32 tensor on device, without waiting for the GPU. Tokens given on the host (arrays,
     lists, CPU tensors) are checked against [0, vocab) there (ValueError, as the reference rejects a bad token file up
@@ -55,14 +74,7 @@ def device_tokens(tokens, vocab: int, device, check_device: bool = False) -> tor
                 (int(x.min()) < 0 or int(x.max()) >= vocab):
             raise ValueError(f"token out of range [0, {vocab})")
         return x
-    a = tokens.numpy() if isinstance(tokens, torch.Tensor) else np.asarray(tokens)
-    if a.dtype.kind not in "iu":
-        raise ValueError(f"tokens must be integers, got {a.dtype}")
-    if not a.dtype.isnative:
-        a = a.astype(a.dtype.newbyteorder("="))
-    # (one pass: a negative entry is a large one as unsigned)
-    if a.size and int(a.view(f"u{a.dtype.itemsize}").max()) >= vocab:
-        raise ValueError(f"token out of range [0, {vocab})")
+    a = host_tokens(tokens, vocab)
     if not a.size:
         return torch.empty(a.shape, dtype=torch.int32, device=device)
     host = torch.empty(a.shape, dtype=torch.int32, pin_memory=True)
