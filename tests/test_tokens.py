@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from yggdrasil_amd import synth
-from yggdrasil_amd.inference import device_tokens, host_tokens
+from yggdrasil_amd.inference import Yggdrasil, device_tokens, host_tokens
 
 TYPES = ["int8", "uint8", "int16", ">i2", "uint16", "int32", ">i4", "uint32", "int64", ">i8", "uint64"]
 
@@ -38,10 +38,18 @@ def test_no_integers(a):
         host_tokens(a, 256)
 
 
+@pytest.mark.parametrize("targets", [False, True])
+def test_score_takes_windows_of_two_axes(targets):
+    """Before any device is touched; a third axis was once read as more of the first rows' tokens."""
+    m = object.__new__(Yggdrasil)
+    a = np.zeros((2, 3, 4), np.int64)
+    with pytest.raises(ValueError, match="tokens must be"):
+        m.score(a, targets=a if targets else None)
+
+
 @pytest.mark.gpu
 def test_calls_refuse_narrow_negative_tokens(tmp_path):
     """run, step and score on int8 arrays, whose -1 has the bits of token 255; the same values as other types pass."""
-    from yggdrasil_amd.inference import Yggdrasil
     p = tmp_path / "m.bin"
     synth.write_model(synth.ModelSpec(64, 16, 4, 256, 2, 8, 16), 3, p)
     m = Yggdrasil.load(p)

@@ -313,6 +313,8 @@ class Yggdrasil:
         out = []
         for i in range(0, len(tokens), batch):
             rows = tokens[i:i + batch]
+            if rows.ndim != 2:
+                raise ValueError(f"tokens must be (B, L), got {tokens.shape}")
             B, T = rows.shape[0], rows.shape[1] - (targets is None)
             st = self.init_state(B) if state is None else self._check_state(state[i:i + B], B).clone()
             nll = torch.zeros(B, dtype=torch.float64, device=self.device)
