@@ -122,6 +122,44 @@ def test_scan_in_chunks_and_bad_tokens(spec, mode, tmp_path, monkeypatch):
     m.close()
 
 
+@pytest.mark.parametrize("score", [0, 1])
+def test_scratch_between_row_by_row_and_sorted(score, tmp_path, monkeypatch):
+    """A call whose rows would be sorted, in scratch for a chunk of a few hundred rows, whose sort's arrays alone are
+    larger: shorter chunks, which are not sorted, and the same bits. 1024 experts: 0.3 MB of sorts' arrays; 60 000 rows,
+    past the 58 594 from which a sort pays at n = 64."""
+    import torch
+    from yggdrasil_amd import _lib
+    from yggdrasil_amd.inference import Yggdrasil
+    monkeypatch.setenv("YGG_SCAN", "1")
+    p = tmp_path / "m.bin"
+    synth.write_model(K(64, 16, 10, 27, 3, 8, 16), 6, p)
+    m, lib = Yggdrasil.load(p), _lib.lib()
+    B, T = 60, 1000
+    x = torch.tensor(np.random.default_rng(7).integers(0, 27, (B, T + 1)), dtype=torch.int32, device=m.device)
+    xd, yd = x[:, :-1].contiguous(), x[:, 1:].contiguous()
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    q = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    least, whole = lib.ygg_scratch(m._h, 60, 2, score), lib.ygg_scratch(m._h, B, T, score)
+    got = []
+    for size in (None, least, least + 100_000, least + 250_000, least + 400_000, whole - 256, whole):
+        st, nll = m.init_state(B), torch.zeros(B, dtype=torch.float64, device=m.device)
+        lg = torch.zeros(B, T, 27, device=m.device)
+        ws = None if size is None else torch.empty(size, dtype=torch.uint8, device=m.device)
+        if score and size is None:
+            rc = lib.ygg_score(m._h, ptr(xd), ptr(yd), B, T, ptr(st), ptr(nll), q)
+        elif score:
+            rc = lib.ygg_score_scratch(m._h, ptr(xd), ptr(yd), B, T, ptr(st), ptr(nll), ptr(ws), size, q)
+        elif size is None:
+            rc = lib.ygg_run(m._h, ptr(xd), B, T, ptr(st), ptr(lg), None, None, None, q)
+        else:
+            rc = lib.ygg_run_scratch(m._h, ptr(xd), B, T, ptr(st), ptr(lg), None, ptr(ws), size, q)
+        assert rc == 0, f"scratch of {size} bytes: {lib.ygg_last_error().decode()}"
+        got.append([t.cpu().numpy() for t in (st, nll, lg)])
+        for a, b in zip(got[0], got[-1]):
+            np.testing.assert_array_equal(a, b)
+    m.close()
+
+
 def test_scan_taken_where_it_pays(tmp_path, monkeypatch):
     """The calls that go layer by layer: long enough ones of few streams, large batches of the trained shapes and every
     factored call, but no call of one token, no short one of a table model and none with a kernel forced."""

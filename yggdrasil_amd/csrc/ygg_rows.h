@@ -40,6 +40,18 @@ inline int64_t sort_fixed_bytes(int64_t N, int E, bool sorted) {
 }
 constexpr int64_t kSortRowBytes = 12 + 1;
 
+// The most rows, at most N, whose workspace fits: need(rows) bytes, more for more rows (a sort's arrays among them from
+// where its rows are sorted on), in `bytes`; 0 if none.
+template <class Need> inline int64_t rows_that_fit(int64_t N, int64_t bytes, Need need) {
+    int64_t lo = 0, hi = N;
+    while (lo < hi) {
+        const int64_t mid = hi - (hi - lo) / 2;
+        if (need(mid) <= bytes) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 template <class Take> inline void lay_out(Sort &s, int N, int E, bool sorted, Take take) {
     s.N = N;
     s.E = E;

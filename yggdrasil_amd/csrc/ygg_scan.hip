@@ -838,18 +838,22 @@ bool sort_pays(const YggDevModel &m, int64_t N) {
 }
 
 struct ScanPlan {
-    int64_t fixed, per_row;
+    int64_t fixed, per_row;      // workspace bytes besides the rows' and the sorts', and per row (arrays rounded up apart)
     int E, ZLW, ZQW;
 };
 
-ScanPlan scan_plan(const YggDevModel &m, int64_t B, int64_t T, bool score, bool sort) {
+ScanPlan scan_plan(const YggDevModel &m, int64_t B, bool score) {
     ScanPlan p{};
     p.E = m.E > m.V ? m.E : m.V;
     p.ZLW = (m.R2 + 15) / 16 * 16;
     p.ZQW = m.L * m.R;
     p.per_row = 4 * (int64_t)m.N + p.ZLW + p.ZQW + 8 + 2 * kSortRowBytes + (score ? 16 : 0);
-    p.fixed = 256 * 12 + B * 4 + (score ? B * 32 : 0) + kPad * (8 + 32) + 2 * sort_fixed_bytes(B * T, p.E, sort || sort_pays(m, B * T));
+    p.fixed = 256 * 12 + B * 4 + (score ? B * 32 : 0) + kPad * (8 + 32);
     return p;
+}
+// workspace bytes of a chunk of N rows, more for more rows
+int64_t scan_bytes(const YggDevModel &m, const ScanPlan &p, int64_t N, bool sort) {
+    return p.fixed + p.per_row * N + 2 * sort_fixed_bytes(N, p.E, sort || sort_pays(m, N));
 }
 
 template <int N, int R, int R2>
@@ -949,18 +953,17 @@ bool scan_pays(const YggDevModel &m, int64_t B, int64_t T) {
 }
 
 int64_t scan_scratch_bytes(const YggDevModel &m, int64_t B, int64_t T, bool score, bool sort, int64_t cap) {
-    const ScanPlan p = scan_plan(m, B, T, score, sort);
-    const int64_t want = p.fixed + p.per_row * B * T, least = p.fixed + p.per_row * 64;
-    cap = std::max(cap, least);
-    return (int64_t)up256((size_t)std::min(want, cap));
+    const ScanPlan p = scan_plan(m, B, score);
+    cap = std::max(cap, scan_bytes(m, p, 64, sort));
+    return (int64_t)up256((size_t)std::min(scan_bytes(m, p, B * T, sort), cap));
 }
 
 hipError_t launch_scan(const YggDevModel &m, const int32_t *tokens, int B, int T, int8_t *state, const YggIO &io,
                        bool group, bool sort, void *ws, int64_t bytes, hipStream_t st) {
     const bool score = io.nll != nullptr;
-    const ScanPlan p = scan_plan(m, B, T, score, sort);
+    const ScanPlan p = scan_plan(m, B, score);
     // a chunk's rows; whole calls where they fit, else runs of at least 128 tokens of as many streams as fit
-    const int64_t rows = (bytes - p.fixed) / p.per_row;
+    const int64_t rows = rows_that_fit((int64_t)B * T, bytes, [&](int64_t N) { return scan_bytes(m, p, N, sort); });
     if (rows < 1) return hipErrorInvalidValue;
     int64_t Tc = T, Bc = B;
     if ((int64_t)B * T > rows) {
