@@ -125,3 +125,31 @@ def test_scan_in_chunks_and_bad_tokens(case, end, few, tol):
         assert (lg[s, t:] == 7.0).all() and (lv[s, t:] == -5).all()
     assert lib.ygg_float_run_scratch(m._h, p[0], B, T, p[1], p[2], p[3], p[4], p[5], 256, None) == 5   # too little
     m.close()
+
+
+def test_scratch_between_row_by_row_and_sorted():
+    """A call whose rows would be sorted (8000 rows of 1024 experts in f64, past the 7400 from which a sort pays at n = 64),
+    in scratch for 15 rows and more, where the sorts' arrays (135 KB) would leave none: shorter chunks, and the step
+    kernel's values (bound as above)."""
+    import torch
+    from yggdrasil_amd import _lib
+    layers, ob = _layers((64, 8, 16, 10, 3, 32, 16, True, 40, 200))
+    m, lib = FM.FloatYggdrasil(layers, ob, precision=64), _lib.lib()
+    B, T, V = 40, 200, 32
+    x = torch.tensor(np.random.default_rng(8).integers(0, V, (B, T)), dtype=torch.int32, device=m.device)
+    q = torch.cuda.current_stream().cuda_stream
+    least, whole = lib.ygg_float_scratch(m._h, 1, 16), lib.ygg_float_scratch(m._h, B, T)
+    got = []
+    for size in (None, least, least + 60_000, least + 130_000, whole - 256, whole):
+        st, lg = m.init_state(B), torch.zeros(B, T, V, dtype=m.dtype, device=m.device)
+        if size is None:
+            rc = lib.ygg_float_run(m._h, x.data_ptr(), B, T, st.data_ptr(), lg.data_ptr(), None, None, q)
+        else:
+            ws = torch.empty(size, dtype=torch.uint8, device=m.device)
+            rc = lib.ygg_float_run_scratch(m._h, x.data_ptr(), B, T, st.data_ptr(), lg.data_ptr(), None, None,
+                                           ws.data_ptr(), size, q)
+        assert rc == 0, f"scratch of {size} bytes: {lib.ygg_last_error().decode()}"
+        got.append((st.cpu().numpy(), lg.cpu().numpy()))
+        for a, b in zip(got[0], got[-1]):
+            np.testing.assert_allclose(b, a, rtol=1e-10, atol=1e-10)
+    m.close()

@@ -669,21 +669,23 @@ constexpr int64_t kSortBytes = 130'000'000;
 bool sort_pays(int64_t N, int E, int64_t record) { return E <= kSortLeaves && N > E && (N - E) * record >= kSortBytes; }
 
 struct Plan {
-    int64_t fixed, per_row;      // workspace bytes besides the rows' and per row (arrays rounded up apart)
-    int E, ZLW, ZW;
+    int64_t fixed, per_row;      // workspace bytes besides the rows' and the sorts', and per row (arrays rounded up apart)
+    int L, E, ZLW, ZW;
     int64_t record;              // bytes of an expert's record
+    // workspace bytes of a chunk of N rows, more for more rows
+    int64_t bytes(int64_t N) const { return fixed + per_row * N + L * sort_fixed_bytes(N, E, sort_pays(N, E, record)); }
 };
 
-template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
+template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B) {
     Plan p{};
+    p.L = m.L;
     const int64_t leaves = m.L > 1 ? (int64_t)1 << m.D : 1;
     p.E = (int)(leaves > m.V ? leaves : m.V);
     p.record = record_bytes(m);
     p.ZLW = (m.R2 + 15) / 16 * 16;
     p.ZW = (m.L * m.R + 15) / 16 * 16;
     p.per_row = (int64_t)sizeof(T) * ((int64_t)m.L * (m.n + p.ZLW) + p.ZW) + 4 + m.L * kSortRowBytes;
-    p.fixed = 256 * 8 + B * 4 + kPad * (4 + (int64_t)m.n * sizeof(T)) +
-              m.L * sort_fixed_bytes(B * Tn, p.E, sort_pays(B * Tn, p.E, p.record));
+    p.fixed = 256 * 8 + B * 4 + kPad * (4 + (int64_t)m.n * sizeof(T));
     return p;
 }
 
@@ -710,10 +712,8 @@ template <typename T> bool takes(const FloatDevModel<T> &m, int64_t B, int64_t T
 
 template <typename T> int64_t scratch_of(const FloatDevModel<T> &m, int64_t B, int64_t Tn) {
     if (!takes(m, B, Tn)) return 0;
-    const Plan p = plan_of(m, B, Tn);
-    const int64_t want = p.fixed + p.per_row * B * Tn, least = p.fixed + p.per_row * 64;
-    const int64_t cap = kScratchCap > least ? kScratchCap : least;
-    return (int64_t)up256(want < cap ? want : cap);
+    const Plan p = plan_of(m, B);
+    return (int64_t)up256(std::min(p.bytes(B * Tn), std::max(kScratchCap, p.bytes(64))));
 }
 
 // Rows below which the route takes two levels a step.
@@ -730,9 +730,9 @@ template <typename T, int EPL> void route_of(const FloatDevModel<T> &m, const Ch
 template <typename T>
 int scan_run(const FloatDevModel<T> &m, const int32_t *tokens, int B, int Tn, T *state, T *logits, int32_t *leaves,
              double *stats, void *scratch, int64_t bytes, hipStream_t st) {
-    const Plan p = plan_of(m, B, Tn);
+    const Plan p = plan_of(m, B);
     // a chunk's rows; whole calls where they fit, else runs of at least 128 tokens of as many streams as fit
-    const int64_t rows = (bytes - p.fixed) / p.per_row;
+    const int64_t rows = rows_that_fit((int64_t)B * Tn, bytes, [&](int64_t N) { return p.bytes(N); });
     if (rows < 1) return fail(YGG_ERR_ARG, "float scratch of %lld bytes is too small", (long long)bytes);
     int64_t Tc = Tn, Bc = B;
     if ((int64_t)B * Tn > rows) {
