@@ -22,7 +22,20 @@ CASES = [
     (128, 16, 32, 11, 2, 20, 7, True, 4),     # three rounds, the last of one level
     (256, 32, 64, 4, 5, 20, 32, True, 3),
     (256, 32, 64, 6, 3, 256, 5, True, 1),
-    (256, 32, 64, 4, 2, 20, 33, True, 3),     # a token part of 33: the general build
+    (256, 32, 64, 4, 2, 20, 33, True, 3),     # a token part of 33, past the plain build's
+]
+# the same shapes where the plain build does not take the call: its token part's remainder at 8, 16 and 32 lanes a node,
+# the widest, no transitions (False), the maxima of a model that the plain build takes
+ANY_CASES = [
+    (64, 8, 16, 6, 3, 33, 33, True, 5, True),
+    (64, 8, 16, 1, 2, 64, 256, False, 3, True),
+    (64, 8, 16, 5, 3, 256, 16, True, 5, False),
+    (128, 16, 32, 11, 2, 20, 71, True, 4, True),
+    (128, 16, 32, 5, 3, 33, 16, False, 4, True),
+    (128, 16, 32, 4, 5, 20, 48, True, 3, False),
+    (256, 32, 64, 6, 3, 256, 256, True, 1, True),
+    (256, 32, 64, 10, 2, 20, 16, True, 3, False),
+    (256, 32, 64, 4, 8, 20, 32, True, 3, True),
 ]
 
 
@@ -75,8 +88,8 @@ def test_step_equals_restatement(case):
     first = FO.run(layers, ob, x[:, :4])
     ref = FO.run(layers, ob, x[:, 4:], state=first["state"])
     m, lib = FM.FloatYggdrasil(layers, ob, precision=32), _lib.lib()
-    assert m.kernel_name == ("ygg::float_kernel<float>" if F > 32 else
-                             "ygg::float_kernel<float, %d, %d, %d, 16>" % (n, R, R2)), m.kernel_name
+    assert m.kernel_name == ("ygg::float_any_kernel<%d, %d, %d>" if F > 32 else
+                             "ygg::float_kernel<float, %d, %d, %d, 16>") % (n, R, R2), m.kernel_name
     end = T - 4 if B == 1 else 9                # the last stream ends at a token outside [0, V)
     if B > 1:
         x[-1, 4 + end] = V
@@ -102,4 +115,48 @@ def test_step_equals_restatement(case):
         if upto == t1 == T - 4:
             np.testing.assert_allclose(st[s], ref["state"][s], rtol=2e-4, atol=2e-4)
     assert split <= 1
+    m.close()
+
+
+@pytest.mark.parametrize("stats", [True, False], ids=["stats", "plain"])
+@pytest.mark.parametrize("case", ANY_CASES, ids=[str(c) for c in ANY_CASES])
+def test_any_build_equals_restatement(case, stats):
+    """The step build of a trained shape for the calls that the plain one does not take; the maxima up to 2e-4 as well,
+    where no route differs."""
+    import torch
+    n, R, R2, D, L, V, F, rs, B, moves = case
+    print(f"case {case} {stats}", flush=True)
+    spec = FM.FloatSpec(d_state=n, block_size=16, router_depth=D, vocab=V, n_layers=L, router_token_dim=F,
+                        input_rank=8, readout_rank=R, layer_input_rank=R2, router_state=rs)
+    p = {k: v for k, v in FM.random_params(spec, 6).items() if moves or k.rsplit("/")[-1] not in ("rotation", "decay")}
+    raw, ob = FM.from_params(p)
+    layers = FM.float_layers(raw)
+    T = 16
+    x = np.random.default_rng(5).integers(0, V, (B, T + 4))
+    first = FO.run(layers, ob, x[:, :4])
+    ref = FO.run(layers, ob, x[:, 4:], state=first["state"])
+    m, lib = FM.FloatYggdrasil(layers, ob, precision=32), _lib.lib()
+    plain = moves and F <= 32
+    assert m.kernel_name == ("ygg::float_kernel<float, %d, %d, %d, 16>" if plain else
+                             "ygg::float_any_kernel<%d, %d, %d>") % (n, R, R2), m.kernel_name
+    st = torch.tensor(first["state"], dtype=m.dtype, device=m.device)
+    xd = torch.tensor(x[:, 4:], dtype=torch.int32, device=m.device).contiguous()
+    lg = torch.empty(B, T, V, dtype=m.dtype, device=m.device)
+    lv = torch.empty(B, T, L, dtype=torch.int32, device=m.device)
+    sv = torch.zeros(L, m.stats_stride, dtype=torch.float64, device=m.device)
+    _lib.check(lib.ygg_float_run(m._h, xd.data_ptr(), B, T, st.data_ptr(), lg.data_ptr(), lv.data_ptr(),
+                                 sv.data_ptr() if stats else None, torch.cuda.current_stream().cuda_stream))
+    lg, lv, st, sv = (t.cpu().numpy() for t in (lg, lv, st, sv))
+    split = 0
+    for s in range(B):
+        d = (lv[s] != ref["leaves"][s]).any(-1)
+        upto = int(np.argmax(d)) if d.any() else T
+        split += upto < T
+        np.testing.assert_allclose(lg[s, :upto], ref["logits"][s, :upto], rtol=2e-4, atol=2e-4)
+        if upto == T:
+            np.testing.assert_allclose(st[s], ref["state"][s], rtol=2e-4, atol=2e-4)
+    assert split <= 1
+    if stats and not split:
+        np.testing.assert_allclose(sv, ref["stats"], rtol=2e-4, atol=0)
+    assert stats or not sv.any()
     m.close()

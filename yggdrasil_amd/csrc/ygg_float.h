@@ -45,17 +45,21 @@ template <typename T> struct FloatDevModel {
     FloatLayerDev<T> layers[YGG_MAX_LAYERS];
 };
 
-// Whether the f32 step of the trained shapes takes a model: of their sizes, with transitions, and at most 32 token entries
-// in a router's input (a lane's loads of a node's row are one of these and 8 of the state's).
-constexpr int kStepF = 32;
+// Whether a model has the f32 step of the trained shapes.
 inline bool float_steps(const FloatDevModel<float> &m) {
-    if (m.b != 16 || (m.L > 1 && m.F > kStepF)) return false;
-    for (int l = 0; l < m.L; l++)
-        if (!m.layers[l].A) return false;
-    return (m.n == 64 && m.R == 8 && m.R2 == 16) || (m.n == 128 && m.R == 16 && m.R2 == 32) ||
-           (m.n == 256 && m.R == 32 && m.R2 == 64);
+    return m.b == 16 && ((m.n == 64 && m.R == 8 && m.R2 == 16) || (m.n == 128 && m.R == 16 && m.R2 == 32) ||
+                         (m.n == 256 && m.R == 32 && m.R2 == 64));
 }
 inline bool float_steps(const FloatDevModel<double> &) { return false; }
+// Whether that step's plain build takes it (calls without maxima): with transitions, and at most 32 token entries in a
+// router's input (a lane's loads of a node's row are one of these and 8 of the state's).
+constexpr int kStepF = 32;
+inline bool step_whole(const FloatDevModel<float> &m) {
+    if (m.L > 1 && m.F > kStepF) return false;
+    for (int l = 0; l < m.L; l++)
+        if (!m.layers[l].A) return false;
+    return true;
+}
 
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 

@@ -102,10 +102,15 @@ __device__ __forceinline__ const float *from(const float *base, uint32_t i) {
     return (const float *)((const char *)base + i * 4u);
 }
 
-template <int N, int R, int R2>
+// The step. ANY: models of these sizes with a token part past kStepF entries (the rest loaded where it is added) or without
+// transitions, and calls with the calibration maxima, kept in LDS by the threads that form the values. A build of its own:
+// the plain one keeps its registers. One token of one stream, n = 64 / 128 / 256 (us; the plain build 16 / 17 / 22, the
+// general kernel 110 to 130): a token part of 64 20 / 20 / 25, no transitions 17 / 18 / 23, with the maxima 21 / 21 / 27; of
+// 256 streams 21 / 24 / 34, 18 / 20 / 31 and 40 / 41 / 47, these last bound by the maxima's additions in memory.
+template <int N, int R, int R2, bool ANY>
 __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const int32_t *__restrict__ tokens, int Tn,
                                            float *__restrict__ state, float *__restrict__ logits,
-                                           int32_t *__restrict__ leaves) {
+                                           int32_t *__restrict__ leaves, double *__restrict__ stats) {
     constexpr int NT = 4 * N, G = N / 8, PARTS = NT / R2, VC = N / PARTS, UK = R2 / 4,
                   PL = 32, PE = N / PL, FE = kStepF / G, QP = NT / 256, RQ = R / QP;
     static_assert(NT / R == PL && PARTS == 16 && RQ == 8, "the trained shapes' proportions");
@@ -113,11 +118,16 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
     __shared__ float bl[N], hn[N];            // rms(h) of the layer below; the new state
     __shared__ float zp[PARTS][R2 + 1], zl[R2], up[4][N], zs[R], red[N / 64], lgp[QP][256];
     __shared__ uint32_t dec[4];               // a round's decisions, a bit per node of its subtree
+    // (ANY) maxima of |h| per 16 coordinates, |zl| and |z| per row
+    constexpr int NM = ANY ? N / 16 + R2 + R : 1;
+    __shared__ float top[ANY ? YGG_MAX_LAYERS : 1][NM];
     const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, L = m.L, V = m.V, C = m.classes, F = m.F, D = m.D;
     const bool rs = m.router_state != 0;
     float *st = state + (size_t)s * L * N;
     for (int i = tid; i < L * N; i += NT) hs[i / N][i % N] = st[i];
     if (tid < 4) dec[tid] = 0u;
+    if constexpr (ANY)
+        for (int i = tid; i < L * NM; i += NT) top[i / NM][i % NM] = 0.0f;
     __syncthreads();
     const int32_t *tok = tokens + (size_t)s * Tn;
     for (int t = 0; t < Tn; t++) {
@@ -146,10 +156,11 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
 #pragma unroll
             for (int k = 0; k < FE; k++) emb[k] = *from(e, min(rl + G * k, F - 1));
         };
+        // the row of this thread's node of a round (lanes past the round's nodes: a row that nobody reads)
+        auto node_of = [&](int root, int h) { return rg < (1 << h) - 1 ? ((root + 1) << kdep) - 1 + path : 0; };
         auto load_round = [&](int l, int root, int h) {
-            const int node = ((root + 1) << kdep) - 1 + path;
-            const int at = rg < (1 << h) - 1 ? node : 0;      // (lanes past the round's nodes: a row that nobody reads)
-            const uint32_t row = (uint32_t)at * (F + (rs ? N : 0));      // (at most 2^20 rows of 288)
+            const int at = node_of(root, h);
+            const uint32_t row = (uint32_t)at * (F + (rs ? N : 0));      // (at most 2^20 rows of 512)
 #pragma unroll
             for (int k = 0; k < FE; k++) wt[k] = *from(m.layers[l].W, row + min(rl + G * k, F - 1));
             const float *ws = rs ? from(m.layers[l].W, row + F + rl) : from(m.layers[l].P, rl);   // (P: not used)
@@ -180,6 +191,10 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
                     float p = 0.0f;
 #pragma unroll
                     for (int k = 0; k < FE; k++) p = rl + G * k < F ? fmaf(emb[k], wt[k], p) : p;
+                    if constexpr (ANY) {
+                        const float *e = y.emb + (size_t)x * F, *wr = y.W + (size_t)node_of(root, h) * (F + (rs ? N : 0));
+                        for (int k = kStepF + rl; k < F; k += G) p = fmaf(e[k], wr[k], p);
+                    }
                     if (rs) {
 #pragma unroll
                         for (int k = 0; k < N / G; k++) p = fmaf(f[k], w[k], p);
@@ -192,6 +207,7 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
 #pragma unroll
                         for (int q = 0; q < PARTS; q++) a[q % 4] += zp[q][tid];
                         zl[tid] = (a[0] + a[1]) + (a[2] + a[3]);
+                        if constexpr (ANY) top[l][N / 16 + tid] = fmaxf(top[l][N / 16 + tid], fabsf(zl[tid]));
                     }
                     const uint32_t bits = dec[rd];
                     int j = 0;
@@ -208,7 +224,9 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
 #pragma unroll
                 for (int k = 0; k < UK; k++) uw[k] = u[k * N];
             }
-            const float4 aw = *(const float4 *)from(y.A + (size_t)r * N * 16, (ui / 16) * 256 + a_index<float>(16, ui % 16, 4 * uq));
+            float4 aw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (!ANY || y.A)
+                aw = *(const float4 *)from(y.A + (size_t)r * N * 16, (ui / 16) * 256 + a_index<float>(16, ui % 16, 4 * uq));
             if (uq == 0) tab = *from(y.table + (l == 0 ? (size_t)x : (size_t)r * V + x) * N, ui);
             const int prow = (uq * N + ui) / PL, pu = ui % PL;
             const float *pr = from(y.P + (size_t)r * R * N, prow * N + pu);
@@ -224,10 +242,12 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
                 for (int k = 0; k < UK; k++) a = fmaf(uw[k], zl[uq * UK + k], a);
             }
             const float *ho = hs[l] + (ui & ~15) + 4 * uq;
-            b = fmaf(aw.x, ho[0], b);
-            b = fmaf(aw.y, ho[1], b);
-            b = fmaf(aw.z, ho[2], b);
-            b = fmaf(aw.w, ho[3], b);
+            if (!ANY || y.A) {
+                b = fmaf(aw.x, ho[0], b);
+                b = fmaf(aw.y, ho[1], b);
+                b = fmaf(aw.z, ho[2], b);
+                b = fmaf(aw.w, ho[3], b);
+            }
             up[uq][ui] = a + b;
             __syncthreads();
             if (tid < N) {
@@ -236,6 +256,10 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
                 hs[l][ui] = h;
                 const float ss = wave_sum(h * h);
                 if (lane == 0) red[tid >> 6] = ss;
+                if constexpr (ANY) {
+                    const float g = group_max_n(fabsf(h), 16);
+                    if ((ui & 15) == 0) top[l][ui / 16] = fmaxf(top[l][ui / 16], g);
+                }
             }
             if (tid < 4) dec[tid] = 0u;
             __syncthreads();
@@ -247,7 +271,10 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
 #pragma unroll
             for (int e = 0; e < PE; e++) z = fmaf(pw[e], hn[pu + PL * e], z);
             z = lanes_sum<PL>(z);
-            if (pu == 0) zs[prow] = z;
+            if (pu == 0) {
+                zs[prow] = z;
+                if constexpr (ANY) top[l][N / 16 + R2 + prow] = fmaxf(top[l][N / 16 + R2 + prow], fabsf(z));
+            }
             __syncthreads();
             float q = 0.0f;
 #pragma unroll
@@ -268,12 +295,35 @@ __device__ __forceinline__ void float_step(const FloatDevModel<float> &m, const 
     }
     __syncthreads();
     for (int i = tid; i < L * N; i += NT) st[i] = hs[i / N][i % N];
+    if constexpr (ANY) {
+        if (stats && tid < 64)
+            for (int l = 0; l < L; l++) {
+                double *to = stats + (size_t)l * (3 + N / 16 + R);
+                const float h = lane < N / 16 ? top[l][lane] : 0.0f, v = lane < R2 ? top[l][N / 16 + lane] : 0.0f,
+                            z = lane < R ? top[l][N / 16 + R2 + lane] : 0.0f;
+                const double ha = wave_max(h), va = wave_max(v), za = wave_max(z);
+                if (lane == 0) {
+                    atomic_max_nonneg(to, ha);
+                    atomic_max_nonneg(to + 1, va);
+                    atomic_max_nonneg(to + 2, za);
+                }
+                if (lane < N / 16) atomic_max_nonneg(to + 3 + lane, h);
+                if (lane < R) atomic_max_nonneg(to + 3 + N / 16 + lane, z);
+            }
+    }
+}
+
+template <int N, int R, int R2>
+__global__ __launch_bounds__(4 * N) __attribute__((amdgpu_waves_per_eu(N / 64, 8))) void float_any_kernel(
+    const FloatDevModel<float> m, const int32_t *__restrict__ tokens, int Tn, float *__restrict__ state,
+    float *__restrict__ logits, int32_t *__restrict__ leaves, double *__restrict__ stats) {
+    float_step<N, R, R2, true>(m, tokens, Tn, state, logits, leaves, stats);
 }
 
 // stats (calibration maxima, cpu/export.py:127-153), per layer: [|h|, |V' rms(h_below)|, |P_r h|, |h| per 16
 // coordinates (n/16), |P_r h| per row (R)]
 // NS, RS, R2S, BS: the state width, readout rank, layer-input rank and block size of a float_step build (the reference's
-// trained shapes; no stats), or 0 for the model's (any shape the loader takes)
+// trained shapes, as step_whole and without stats), or 0 for the model's (any shape the loader takes)
 // (one wavefront per SIMD: the unrolled row loads of a thread are its registers)
 template <typename T, int NS = 0, int RS = 0, int R2S = 0, int BS = 0>
 __global__ __launch_bounds__(NS ? 4 * NS : kFThreads)
@@ -281,7 +331,7 @@ __attribute__((amdgpu_waves_per_eu(NS ? NS / 64 : 1, NS ? 8 : 1))) void float_ke
     const FloatDevModel<T> m, const int32_t *__restrict__ tokens, int Tn, T *__restrict__ state,
     T *__restrict__ logits, int32_t *__restrict__ leaves, double *__restrict__ stats) {
     if constexpr (NS != 0) {
-        float_step<NS, RS, R2S>(m, tokens, Tn, state, logits, leaves);
+        float_step<NS, RS, R2S, false>(m, tokens, Tn, state, logits, leaves, nullptr);
         return;
     } else {
     constexpr int MN = kMaxN, MR = kMaxR, MR2 = kMaxR2, MB = kMaxB;
@@ -668,11 +718,11 @@ int ygg_float_run(const ygg_fmodel *m, const int32_t *d_tokens, int B, int T, vo
             hipLaunchKernelGGL(kernel, dim3(B), dim3(threads), 0, (hipStream_t)stream, fm, d_tokens, T,
                                (float *)d_state, (float *)d_logits, d_leaves, d_stats);
         };
-        const bool step = float_steps(fm) && !d_stats;
-        if (step && fm.n == 64) go(float_kernel<float, 64, 8, 16, 16>, 256);
-        else if (step && fm.n == 128) go(float_kernel<float, 128, 16, 32, 16>, 512);
-        else if (step && fm.n == 256) go(float_kernel<float, 256, 32, 64, 16>, 1024);
-        else go(float_kernel<float>, kFThreads);
+        const bool any = d_stats || !step_whole(fm);
+        if (!float_steps(fm)) go(float_kernel<float>, kFThreads);
+        else if (fm.n == 64) any ? go(float_any_kernel<64, 8, 16>, 256) : go(float_kernel<float, 64, 8, 16, 16>, 256);
+        else if (fm.n == 128) any ? go(float_any_kernel<128, 16, 32>, 512) : go(float_kernel<float, 128, 16, 32, 16>, 512);
+        else any ? go(float_any_kernel<256, 32, 64>, 1024) : go(float_kernel<float, 256, 32, 64, 16>, 1024);
     } else
         hipLaunchKernelGGL(float_kernel<double>, dim3(B), dim3(kFThreads), 0, (hipStream_t)stream, m->m64, d_tokens, T,
                            (double *)d_state, (double *)d_logits, d_leaves, d_stats);

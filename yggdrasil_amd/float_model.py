@@ -256,11 +256,14 @@ class FloatYggdrasil:
         self._h = h
         self.output_bias = np.asarray(output_bias, np.float64)
         # the build ygg_float_run launches (csrc/ygg_float.hip: f32 builds of their own for the reference's trained
-        # shapes (n, R, R2) at block 16 with transitions, else the general one), as profilers name it
+        # shapes (n, R, R2) at block 16, one for models with transitions and at most 32 token entries in a router's
+        # input, called without stats, and one for the others; else the general one), as profilers name it
         shape = (self.n, R, R2)
-        if (precision == 32 and d.block_size == 16 and shape in ((64, 8, 16), (128, 16, 32), (256, 32, 64))
-                and all(y.transition is not None for y in layers) and (len(layers) == 1 or d.router_token_dim <= 32)):
-            self.kernel_name = "ygg::float_kernel<float, %d, %d, %d, 16>" % shape
+        if precision == 32 and d.block_size == 16 and shape in ((64, 8, 16), (128, 16, 32), (256, 32, 64)):
+            if all(y.transition is not None for y in layers) and (len(layers) == 1 or d.router_token_dim <= 32):
+                self.kernel_name = "ygg::float_kernel<float, %d, %d, %d, 16>" % shape
+            else:
+                self.kernel_name = "ygg::float_any_kernel<%d, %d, %d>" % shape
         else:
             self.kernel_name = "ygg::float_kernel<%s>" % ("float" if precision == 32 else "double")
 
