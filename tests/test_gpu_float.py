@@ -1,4 +1,5 @@
-"""GPU: the float step (csrc/ygg_float.hip through ygg_float_run) against the float64 restatement oracle/float_oracle.py,
+"""GPU: the float step (csrc/ygg_float.hip through ygg_float_run) and, through FloatYggdrasil.run, whichever form that
+takes (csrc/ygg_float_scan.hip from a few tokens on), against the float64 restatement oracle/float_oracle.py,
 and the int8 export (yggdrasil_amd.export) whose calibration runs on the f64 kernel and whose margin search runs the
 int8 kernel.
 
@@ -14,6 +15,7 @@ import numpy as np
 import pytest
 
 from oracle import float_oracle as FO
+from yggdrasil_amd import _lib
 from yggdrasil_amd import float_model as FM
 
 pytestmark = pytest.mark.gpu
@@ -38,14 +40,37 @@ def _tokens(B, T, seed):
     return np.random.default_rng(seed).integers(0, SPEC.vocab, (B, T))
 
 
-def test_float64_kernel_equals_restatement(ckpt):
+def _run(m, x, form, stats=False):
+    """x through m from the zero state: leaves, logits, state and maxima, in the form named."""
     import torch
+    B, T = x.shape
+    lib = _lib.lib()
+    if form == "layer by layer":
+        assert lib.ygg_float_scratch(m._h, B, T) > 0
+        r = m.run(x, leaves=True, stats=stats)
+    else:
+        xd = torch.tensor(x, dtype=torch.int32, device=m.device)
+        r = dict(state=m.init_state(B), logits=torch.empty(B, T, m.classes, dtype=m.dtype, device=m.device),
+                 leaves=torch.empty(B, T, m.layers, dtype=torch.int32, device=m.device))
+        if stats:
+            r["stats"] = torch.zeros(m.layers, m.stats_stride, dtype=torch.float64, device=m.device)
+        _lib.check(lib.ygg_float_run(m._h, xd.data_ptr(), B, T, r["state"].data_ptr(), r["logits"].data_ptr(),
+                                     r["leaves"].data_ptr(), r["stats"].data_ptr() if stats else None,
+                                     torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return r
+
+
+both_forms = pytest.mark.parametrize("form", ["token by token", "layer by layer"])
+
+
+@both_forms
+def test_float64_kernel_equals_restatement(ckpt, form):
     p, layers, ob = ckpt
     x = _tokens(16, 40, 1)
     ref = FO.run(layers, ob, x)
     m = FM.FloatYggdrasil(layers, ob, precision=64)
-    r = m.run(x, leaves=True, stats=True)
-    torch.cuda.synchronize()
+    r = _run(m, x, form, stats=True)
     np.testing.assert_array_equal(r["leaves"].cpu().numpy(), ref["leaves"])
     np.testing.assert_allclose(r["logits"].cpu().numpy(), ref["logits"], rtol=1e-10, atol=1e-10)
     np.testing.assert_allclose(r["state"].cpu().numpy(), ref["state"], rtol=1e-10, atol=1e-10)
@@ -53,14 +78,13 @@ def test_float64_kernel_equals_restatement(ckpt):
     m.close()
 
 
-def test_float32_kernel_close_to_restatement(ckpt):
-    import torch
+@both_forms
+def test_float32_kernel_close_to_restatement(ckpt, form):
     p, layers, ob = ckpt
     x = _tokens(64, 48, 2)
     ref = FO.run(layers, ob, x)
     m = FM.FloatYggdrasil(layers, ob, precision=32)
-    r = m.run(x, leaves=True)
-    torch.cuda.synchronize()
+    r = _run(m, x, form)
     lv, lg = r["leaves"].cpu().numpy(), r["logits"].cpu().numpy().astype(np.float64)
     differs = (lv != ref["leaves"]).any(-1)            # (B, T): some layer took another leaf
     split = 0
@@ -73,13 +97,13 @@ def test_float32_kernel_close_to_restatement(ckpt):
     m.close()
 
 
-@pytest.mark.parametrize("shape", [(128, 16, 32), (256, 32, 64)], ids=["medium", "large"])
-def test_float32_trained_shape_builds(shape):
-    """The f32 builds specialised on the reference's medium and large trained shapes (5 layers, block 16, router depth
-    10: rounds of 4, 4 and 2 levels, the first from LDS; configs/enwik8/{medium,large}.yaml), against the float64
-    restatement as in test_float32_kernel_close_to_restatement. A vocabulary of 32 keeps the precomputed tables small
-    (the build is picked by the shape alone)."""
-    import torch
+@both_forms
+@pytest.mark.parametrize("shape", [(64, 8, 16), (128, 16, 32), (256, 32, 64)], ids=["small", "medium", "large"])
+def test_float32_trained_shape_builds(shape, form):
+    """The f32 builds specialised on the reference's trained shapes (5 layers, block 16, router depth 10: two rounds of 5
+    levels; configs/enwik8/{small,medium,large}.yaml), and the layer-by-layer form on them, against the float64 restatement
+    as in test_float32_kernel_close_to_restatement. A vocabulary of 32 keeps the precomputed tables small (the build is
+    picked by the shape)."""
     n, R, R2 = shape
     spec = FM.FloatSpec(d_state=n, block_size=16, router_depth=10, vocab=32, n_layers=5, router_token_dim=16,
                         input_rank=64 if n == 256 else 32, readout_rank=R, layer_input_rank=R2)
@@ -89,9 +113,8 @@ def test_float32_trained_shape_builds(shape):
     ref = FO.run(layers, ob, x)
     m = FM.FloatYggdrasil(layers, ob, precision=32)
     assert m.kernel_name == "ygg::float_kernel<float, %d, %d, %d, 16>" % shape, m.kernel_name
-    _say(f"trained shape {shape}: {m.kernel_name}")
-    r = m.run(x, leaves=True)
-    torch.cuda.synchronize()
+    _say(f"trained shape {shape}: {m.kernel_name if form == 'token by token' else form}")
+    r = _run(m, x, form)
     lv, lg = r["leaves"].cpu().numpy(), r["logits"].cpu().numpy().astype(np.float64)
     differs = (lv != ref["leaves"]).any(-1)
     split = 0

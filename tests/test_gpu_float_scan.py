@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from oracle import float_oracle as FO
+from yggdrasil_amd import _lib
 from yggdrasil_amd import float_model as FM
 
 pytestmark = pytest.mark.gpu
@@ -19,7 +20,7 @@ pytestmark = pytest.mark.gpu
 # n, R, R2, depth, layers, vocab, token part, state in the router, streams, tokens
 CASES = [
     (64, 8, 16, 5, 3, 64, 16, True, 7, 33),      # one row per tile, as in all but the last four
-    (64, 8, 16, 10, 3, 32, 16, True, 3, 5),      # more experts than rows
+    (64, 8, 16, 10, 3, 32, 16, True, 3, 16),     # more experts than rows
     (16, 5, 0, 3, 2, 27, 10, True, 5, 9),        # one block, no layer input, a token part of no whole vector
     (48, 3, 20, 4, 2, 5, 4, True, 9, 17),        # three blocks, a layer input of 20
     (96, 8, 7, 6, 3, 30, 16, False, 4, 70),      # routing on the token alone, a layer input of 7, 30 classes
@@ -58,6 +59,7 @@ def test_scan_equals_restatement(case):
     for precision, tol in ((64, 1e-10), (32, 2e-4)):
         m = FM.FloatYggdrasil(layers, ob, precision=precision)
         st = torch.tensor(first["state"], device=m.device)
+        assert _lib.lib().ygg_float_scratch(m._h, B, T - T // 2) > 0        # (else the step kernel runs)
         r = m.run(x[:, T // 2:], state=st, leaves=True, stats=True)
         torch.cuda.synchronize()
         lv = r["leaves"].cpu().numpy()
@@ -83,7 +85,6 @@ def test_scan_in_chunks_and_bad_tokens(case, end, few, tol):
     first and in a later chunk, in the last token and at once: their state is the one before it and their later rows are
     left as they were; and the same call with whole scratch gives the same values (bits, where both sort alike)."""
     import torch
-    from yggdrasil_amd import _lib
     layers, ob = _layers(case)
     B, T, V = case[8], case[9], case[5]
     x = np.random.default_rng(2).integers(0, V, (B, T))
@@ -132,7 +133,6 @@ def test_scratch_between_row_by_row_and_sorted():
     in scratch for 15 rows and more, where the sorts' arrays (135 KB) would leave none: shorter chunks, and the step
     kernel's values (bound as above)."""
     import torch
-    from yggdrasil_amd import _lib
     layers, ob = _layers((64, 8, 16, 10, 3, 32, 16, True, 40, 200))
     m, lib = FM.FloatYggdrasil(layers, ob, precision=64), _lib.lib()
     B, T, V = 40, 200, 32
