@@ -690,12 +690,16 @@ template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B) {
 }
 
 // Calls of fewer than 4 tokens stay on the step kernel, and so do transition blocks other than 16. A model without a
-// step build of its own comes here from 4 tokens: the general step took, at 4 tokens of 1 / 16 / 256 / 1024 streams (us,
-// step / this form), small 132/77, 134/84, 135/98, 531/177; medium 148/90, 151/95, 161/127, 629/214; large 189/113,
-// 193/148, 219/227, 837/387. With one (float_steps) the cheaper is estimated: a step's tokens, by rounds of the streams
-// that fit the chip, against this form's launches, the records its rows read (1.2 TB/s) and the sort. Measured at 4 and 8
-// tokens: small, 1 stream 54/75 104/77, 256 58/96 112/105, 1024 71/150 139/169; medium 57/90 109/91, 76/125 146/146,
-// 152/190 295/248; large 87/115 182/117, 121/230 230/326, 455/388 892/435.
+// step build of its own comes here from 4 tokens, where this form is far ahead of the general kernel: 4 tokens of 1 / 16 /
+// 256 / 1024 streams took (us, general kernel / this form), at depth 10 and 5 layers, n = 64, R = 12, R2 = 16 in f32 409/75
+// 417/85 412/97 1635/129; n = 256, R = R2 = 32 in f32 463/110 471/135 479/189 1905/354, in f64 506/135 513/166 525/327
+// 2078/491; n = 256, R = R2 = 64, 8 layers of depth 6, f64 852/266 865/343 887/507 3508/731; n = 16, 2 layers of depth 3, f32 105/24
+// 108/27 107/29 420/31; a token layer alone, n = 64, f64 55/15 55/19 57/19 218/24. (Fewer tokens were not compared.)
+// With a step build (float_steps) the cheaper is estimated: a step's tokens, by rounds of the streams that fit the chip,
+// against this form's launches, the records its rows read (1.2 TB/s) and the sort. Measured at 4 and 8 tokens: small,
+// 1 stream 54/75 104/77, 256 58/96 112/105, 1024 71/150 139/169; medium 57/90 109/91, 76/125 146/146, 152/190 295/248;
+// large 87/115 182/117, 121/230 230/326, 455/388 892/435. (The step's build for the calls that its plain one does not take
+// is up to a third slower for one stream; the maxima cost both forms.)
 constexpr int kScanTokens = 4;
 constexpr int64_t kScratchCap = (int64_t)1 << 30;
 
