@@ -63,6 +63,7 @@ template <int CTRL> __device__ __forceinline__ float dpp_f32(float v) {
 __device__ __forceinline__ float lane_f32(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
+// the lanes whose pred holds, as a wavefront-uniform 64-bit mask
 __device__ __forceinline__ unsigned long long lane_mask(bool pred) { return __builtin_amdgcn_ballot_w64(pred); }
 // fmaxf over the wavefront (every lane active), returned to every lane: DPP within rows of 16 lanes (quad swaps, the
 // half-row and row mirrors), then the four row maxima from scalar reads. fmaxf ignores NaNs and is exact, so the order
@@ -326,8 +327,6 @@ __device__ __forceinline__ int walk_bits(unsigned long long mask, int h) {
         : "scc");
     return (int)((l + 1) >> (4 - h)) - 1;
 }
-
-// the lanes whose pred holds, as a wavefront-uniform 64-bit mask
 
 // _mm512_cvtps_epi32 in round-to-nearest-even: NaN and |x| >= 2^31 give INT32_MIN (cpu/ygg.cpp:292 and others)
 __device__ __forceinline__ int cvt_rne(float x) {

@@ -199,8 +199,8 @@ def windows(ids, seq_len: int, m: int):
 
 def int8_bits(quant, output_bias, x: np.ndarray, y: np.ndarray, router_token_dim: int, input_rank: int) -> float:
     """Bits per prediction of y (S, T) given x (S, T) under the int8 model `quant`, every window from the zero
-    state, scored on the GPU in one fused launch per 1024 windows (the reference scores int_forward's logits of x
-    against y, cpu/export.py:554-561)."""
+    state, scored on the GPU by 1024 windows (the reference scores int_forward's logits of x against y,
+    cpu/export.py:554-561)."""
     from .inference import Yggdrasil
     with tempfile.TemporaryDirectory() as tmp:
         p = Path(tmp) / "cand.bin"

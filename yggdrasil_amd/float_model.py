@@ -298,8 +298,9 @@ class FloatYggdrasil:
         return device_tokens(tokens, self.vocab, self.device)
 
     def run(self, tokens, state=None, logits: bool = True, leaves: bool = False, stats: bool = False) -> dict:
-        """T tokens per stream in one launch: tokens (B, T) -> dict(state, logits (B, T, classes), leaves (B, T, L),
-        stats (L, 3 + n/16 + R) float64 maxima for calibration)."""
+        """T tokens per stream in one call: tokens (B, T) -> dict(state, logits (B, T, classes), leaves (B, T, L),
+        stats (L, 3 + n/16 + R) float64 maxima for calibration). One launch token by token, or, where ygg_float_scratch
+        gives it scratch, a few launches a layer over the whole call, with up to 1 GiB held for its duration."""
         import torch
         x = self._tokens(tokens)
         if x.dim() != 2:

@@ -34,9 +34,9 @@ def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
 
-def _stream(device: Optional[int] = None):
-    """The current stream of device (default: the current device) as the pointer the C-ABI takes."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device is None else device)
+def _stream():
+    """The current device's current stream as the pointer the C-ABI takes."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def host_tokens(tokens, vocab: int) -> np.ndarray:
@@ -243,9 +243,12 @@ class Yggdrasil:
 
     def run(self, tokens, state: Optional[torch.Tensor] = None, logits: bool = True, leaves: bool = False,
             states: bool = False, digest=False, _entry: str = "ygg_run") -> dict:
-        """T tokens per stream in one launch: tokens (B, T) from state (default zero; not modified) ->
+        """T tokens per stream in one call: tokens (B, T) from state (default zero; not modified) ->
         dict(state=(B, layers, n) after the last token, logits=(B, T, classes), leaves=(B, T, layers) int32,
         states=(B, T, layers, n) int8, digest=(B,) int64 bit pattern of the uint64 digest).
+
+        One launch token by token, or (without states and digest, where ygg_scratch says that it is faster) a few
+        launches a layer over the whole call, with up to 512 MiB of device memory held for its duration.
 
         Tokens given on the host are range-checked before the launch (ValueError). Tokens already on the GPU are not
         read back: a stream whose token t lies outside [0, vocab) stops there, its state stays the one before token
@@ -300,8 +303,8 @@ class Yggdrasil:
         """Bits of tokens[:, 1:] given the tokens before them, per row of tokens (B, L), as float64 (B,); with
         targets (B, L), bits of targets[:, t] given tokens[:, :t + 1] (every token an input, as the reference scores
         windows x against their next tokens y). Rows start from state, or from zero (yggdrasil/inference.py:179-188).
-        One fused launch per batch of rows: the step and the float64 log-softmax of the reference's score mode
-        (cpu/ygg.cpp:513-516), no logits written."""
+        Per batch of rows the step and the float64 log-softmax of the reference's score mode (cpu/ygg.cpp:513-516), no
+        logits written: one fused launch, or layer by layer as in run()."""
         def rows_of(a):
             a = np.asarray(a)
             return np.atleast_2d(a if a.dtype.kind in "iu" else a.astype(np.int64))
@@ -339,8 +342,8 @@ class Yggdrasil:
                  return_logits: bool = False):
         """Prompt (L,) or (B, L), L >= 1, followed by n sampled tokens. temperature 0: greedy
         (yggdrasil/inference.py:190-202, yggdrasil/inference_triton.py:229-248). The prompt but its last token goes
-        through one ygg_run launch; the n sampled tokens come from one ygg_generate launch that samples on the device
-        and feeds each token back as the next input. Draws depend on (seed, row, position) only, so a row samples the
+        through run(); the n sampled tokens come from one ygg_generate launch that samples on the device and feeds each
+        token back as the next input. Draws depend on (seed, row, position) only, so a row samples the
         same tokens whatever the batch around it. return_logits: also the logits (B, n, classes) each token was
         sampled from."""
         prompt = np.asarray(prompt, np.int64)
