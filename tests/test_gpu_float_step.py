@@ -160,3 +160,23 @@ def test_any_build_equals_restatement(case, stats):
         np.testing.assert_allclose(sv, ref["stats"], rtol=2e-4, atol=0)
     assert stats or not sv.any()
     m.close()
+
+
+@pytest.mark.parametrize("precision,tol", [(32, 2e-4), (64, 1e-10)])
+@pytest.mark.parametrize("n,b", [(16, 1), (32, 2), (48, 4), (64, 8), (96, 16), (48, 3)])
+def test_general_kernel_blocks(n, b, precision, tol):
+    """The general kernel's transition blocks of each size, in the layouts that f32 and f64 store them in (bounds as
+    above, 1e-10 in f64)."""
+    spec = FM.FloatSpec(d_state=n, block_size=b, router_depth=3, vocab=20, n_layers=2, router_token_dim=8, input_rank=8,
+                        readout_rank=5, layer_input_rank=7)
+    raw, ob = FM.from_params(FM.random_params(spec, 8))
+    layers = FM.float_layers(raw)
+    x = np.random.default_rng(6).integers(0, 20, (4, 3))
+    ref = FO.run(layers, ob, x)
+    m = FM.FloatYggdrasil(layers, ob, precision=precision)
+    r = m.run(x, leaves=True)
+    lv = r["leaves"].cpu().numpy()
+    np.testing.assert_array_equal(lv, ref["leaves"])
+    np.testing.assert_allclose(r["logits"].cpu().numpy(), ref["logits"], rtol=tol, atol=tol)
+    np.testing.assert_allclose(r["state"].cpu().numpy(), ref["state"], rtol=tol, atol=tol)
+    m.close()

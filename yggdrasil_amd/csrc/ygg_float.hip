@@ -479,8 +479,10 @@ __attribute__((amdgpu_waves_per_eu(NS ? NS / 64 : 1, NS ? 8 : 1))) void float_ke
                 T uw[MR2], aw[MB];
 #pragma unroll
                 for (int k = 0; k < MR2; k++) uw[k] = (up && k < R2) ? u[(size_t)k * n] : T(0);
-                if (ta && b == 16) {     // (whole 16-byte chunks of row ii)
-                    constexpr int VE = 16 / (int)sizeof(T);
+                // (a_index: in f32 whole 16-byte chunks of row ii for b = 16; in f64 they spilled 28 registers more beside the
+                // other layout's loads, 3 to 8% of a token, so there either layout's entries are loaded by strides)
+                constexpr int VE = 16 / (int)sizeof(T);
+                if (sizeof(T) == 4 && ta && b == 16) {
                     struct alignas(16) Chunk { T v[VE]; };
 #pragma unroll
                     for (int j = 0; j < MB / VE; j++) {
@@ -489,8 +491,11 @@ __attribute__((amdgpu_waves_per_eu(NS ? NS / 64 : 1, NS ? 8 : 1))) void float_ke
                         for (int e = 0; e < VE; e++) aw[j * VE + e] = w.v[e];
                     }
                 } else {
+                    const bool chunks = sizeof(T) == 8 && b == 16;
+                    const T *arow = ta ? ablk + (chunks ? ii * VE : ii) : nullptr;
+                    const int chunk = VE * b, next = chunks ? 1 : b;
 #pragma unroll
-                    for (int j = 0; j < MB; j++) aw[j] = (ta && j < b) ? ablk[a_index<T>(b, ii, j)] : T(0);
+                    for (int j = 0; j < MB; j++) aw[j] = (ta && j < b) ? arow[j / VE * chunk + j % VE * next] : T(0);
                 }
                 T h = trow[i];
                 if (up) {
