@@ -150,9 +150,9 @@ int ygg_score(const ygg_model *m, const int32_t *d_tokens, const int32_t *d_targ
    all tokens are known, so only the transition inside a layer is sequential, and an expert's other weights are read once
    for all the rows that take it. The same arguments and results, bit for bit; no counterpart in the reference. d_scratch:
    device memory of scratch_bytes, 256-byte aligned, that no other call uses until this one has run. ygg_scratch gives
-   the bytes a call wants (score: of ygg_score_scratch; at most 512 MiB or 64 rows' worth; with less the call goes in more
-   and shorter chunks), or 0 where the token-by-token call is the faster or the only one: the two calls then take that way
-   and need no scratch. Environment, read at load: YGG_SCAN=0 never, YGG_SCAN=1 every call of at least 2 tokens (of the shapes
+   the bytes a call wants (score 1: of ygg_score_scratch; 0: of ygg_run_scratch; 2: of that without d_logits; at most 512
+   MiB or 64 rows' worth; with less the call goes in more and shorter chunks), or 0 where the token-by-token call is the
+   faster or the only one: the two calls then take that way and need no scratch. Environment, read at load: YGG_SCAN=0 never, YGG_SCAN=1 every call of at least 2 tokens (of the shapes
    that have it), YGG_SCAN=sort the same with the rows always grouped by expert. */
 int64_t ygg_scratch(const ygg_model *m, int B, int T, int score);
 int ygg_run_scratch(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d_state, float *d_logits,

@@ -161,8 +161,8 @@ def test_scratch_between_row_by_row_and_sorted(score, tmp_path, monkeypatch):
 
 
 def test_scan_taken_where_it_pays(tmp_path, monkeypatch):
-    """The calls that go layer by layer: long enough ones of few streams, large batches of the trained shapes and every
-    factored call, but no call of one token, no short one of a table model and none with a kernel forced."""
+    """The calls that go layer by layer: long enough ones of few streams, large batches of the trained shapes and all but
+    the shortest factored calls, but no call of one token, no short one of a table model and none with a kernel forced."""
     from yggdrasil_amd import _lib
     from yggdrasil_amd.inference import Yggdrasil
     p, f = tmp_path / "m.bin", tmp_path / "f.bin"
@@ -175,6 +175,18 @@ def test_scan_taken_where_it_pays(tmp_path, monkeypatch):
     assert not takes(m, 1, 1) and not takes(m, 1, 16) and not takes(m, 256, 32) and not takes(mf, 8, 1)
     m.close()
     mf.close()
+    # short calls of few layers stay token by token at any number of streams (us token by token / layer by layer: 4096 x 2
+    # tokens of the two 128-wide layers 13 / 87, 256 x 8 18 / 24, 256 x 4 of the factored ones 18 / 27)
+    for spec, no, yes in ((K(128, 16, 12, 32, 2, 8, 16), ((1, 2), (4096, 2), (256, 8), (1500, 16)), ((1, 256), (64, 256))),
+                          (K(64, 16, 6, 64, 2, 8, 16, input_rank=32), ((1, 2), (256, 4), (4096, 6)), ((1, 16), (64, 64))),
+                          (K(256, 16, 5, 27, 2, 32, 64), ((1, 4), (4096, 4), (700, 12)), ((4, 48), (64, 64)))):
+        synth.write_model(spec, 7, p)
+        m = Yggdrasil.load(p)
+        for B, T in no:
+            assert not takes(m, B, T) and not lib.ygg_scratch(m._h, B, T, 1), (spec, B, T)
+        for B, T in yes:
+            assert takes(m, B, T) and lib.ygg_scratch(m._h, B, T, 1) and lib.ygg_scratch(m._h, B, T, 2), (spec, B, T)
+        m.close()
     monkeypatch.setenv("YGG_KERNEL", "fast")
     m = Yggdrasil.load(p)
     assert not takes(m, 1, 1024)

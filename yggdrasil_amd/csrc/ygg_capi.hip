@@ -912,9 +912,14 @@ const ygg::Kernel &pick(const ygg_model *m, int B, int T, int mode) {
 
 
 // The calls the layer-by-layer form takes.
-bool scan_takes(const ygg_model *m, int B, int T) {
+bool scan_takes(const ygg_model *m, int B, int T, ygg::ScanCall call) {
     if (!m->scan_ok || B < 1 || T < 2) return false;
-    return m->scan_all || ygg::scan_pays(m->dev, B, T);
+    if (m->scan_all) return true;
+    const ygg::Kernel &k = pick(m, B, T, call == ygg::ScanCall::score ? kModeScore : kModeRun);
+    const ygg::TokenKernel token = &k == &m->flow ? ygg::TokenKernel::flow
+                                   : &k == &m->pipe || &k == &m->pipe_few ? ygg::TokenKernel::pipe
+                                                                          : ygg::TokenKernel::stream;
+    return ygg::scan_pays(m->dev, B, T, call, token);
 }
 constexpr int64_t kScanScratchCap = (int64_t)1 << 29;
 
@@ -1004,15 +1009,18 @@ int ygg_run(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d
 }
 
 int64_t ygg_scratch(const ygg_model *m, int B, int T, int score) {
-    if (!m || !scan_takes(m, B, T)) return 0;
-    return ygg::scan_scratch_bytes(m->dev, B, T, score != 0, m->scan_sort, kScanScratchCap);
+    const ygg::ScanCall call = score == 2 ? ygg::ScanCall::state : (score ? ygg::ScanCall::score : ygg::ScanCall::run);
+    if (!m || !scan_takes(m, B, T, call)) return 0;
+    return ygg::scan_scratch_bytes(m->dev, B, T, call == ygg::ScanCall::score, m->scan_sort, kScanScratchCap);
 }
 
 int ygg_run_scratch(const ygg_model *m, const int32_t *d_tokens, int B, int T, int8_t *d_state, float *d_logits,
                     int32_t *d_leaves, void *d_scratch, int64_t scratch_bytes, void *stream) {
     if (!m) return fail(YGG_ERR_ARG, "model is NULL");
     if (B < 0 || T < 0) return fail(YGG_ERR_ARG, "negative B (%d) or T (%d)", B, T);
-    if (!scan_takes(m, B, T))
+    // (without logits the caller may have asked ygg_scratch for a run with them and got none)
+    if (!scan_takes(m, B, T, d_logits ? ygg::ScanCall::run : ygg::ScanCall::state) ||
+        (!d_scratch && !scan_takes(m, B, T, ygg::ScanCall::run)))
         return ygg_run(m, d_tokens, B, T, d_state, d_logits, d_leaves, nullptr, nullptr, stream);
     if (!d_state || !d_tokens) return fail(YGG_ERR_ARG, "tokens or state is NULL");
     if (!d_scratch || (uintptr_t)d_scratch % 256) return fail(YGG_ERR_ARG, "scratch is NULL or not on 256 bytes");
@@ -1032,7 +1040,7 @@ int ygg_score_scratch(const ygg_model *m, const int32_t *d_tokens, const int32_t
                       int8_t *d_state, double *d_nll, void *d_scratch, int64_t scratch_bytes, void *stream) {
     if (!m) return fail(YGG_ERR_ARG, "model is NULL");
     if (B < 0 || T < 0) return fail(YGG_ERR_ARG, "negative B (%d) or T (%d)", B, T);
-    if (!scan_takes(m, B, T)) return ygg_score(m, d_tokens, d_targets, B, T, d_state, d_nll, stream);
+    if (!scan_takes(m, B, T, ygg::ScanCall::score)) return ygg_score(m, d_tokens, d_targets, B, T, d_state, d_nll, stream);
     if (!d_state || !d_nll || !d_tokens || !d_targets) return fail(YGG_ERR_ARG, "NULL buffer");
     if (!d_scratch || (uintptr_t)d_scratch % 256) return fail(YGG_ERR_ARG, "scratch is NULL or not on 256 bytes");
     if (scratch_bytes < ygg::scan_scratch_bytes(m->dev, B, 1, true, m->scan_sort, 0))

@@ -27,6 +27,9 @@
 // States and inputs pass between the kernels by block, [n / 16][row][16]: a scan's wavefront works on one block, so that an
 // XCD (workgroups go to the XCDs in turn) meets one block's share of every expert's A16, an eighth of them at n = 128, and
 // writes whole lines.
+#include <algorithm>
+#include <cmath>
+
 #include "ygg_kernel_fast.h"
 #include "ygg_launch.h"
 #include "ygg_rows.h"
@@ -935,21 +938,43 @@ template <int R> void scan_logits_of(const YggDevModel &m, const ScanChunk &c, h
 
 }  // namespace
 
-bool scan_pays(const YggDevModel &m, int64_t B, int64_t T) {
-    const double L = m.L, N = (double)B * T, K = (double)m.N * (32 + m.R + m.R2 + m.K) / 1024;
-    // the launches, the recurrence's steps and the rows
-    double scan = 0.067 * L * T;
-    if (sort_pays(m, B * T)) {
-        // (past 4 MB of A16 an XCD's blocks outgrow its L2)
-        const double miss = (double)m.E * m.N * 4 > 6e6 ? 0.5 : 0.0;
-        scan += (m.E > 4096 ? 42 : 28) * L + 1e-3 * N * ((L - 1) * (0.1 + 0.085 * K + miss) + 0.4);
+bool scan_pays(const YggDevModel &m, int64_t B, int64_t T, ScanCall call, TokenKernel token) {
+    // K: KiB of an expert's A16, U', U_r and P; hot: a layer's of these fit an XCD's L2
+    const double L = m.L, P = m.n_rounds, N = (double)B * T, n = m.N, K = n * (32 + m.R + m.R2 + m.K) / 1024;
+    const double score = call == ScanCall::score, out = call != ScanCall::state;
+    const bool hot = m.E * K <= 4096;
+    // token by token: a stream's tokens one after the other while the streams do not fill the chip, then all rows
+    double alone, rows;
+    if (m.K) {
+        alone = L * (1.3 + T * (0.52 + 0.086 * K + 0.51 * P + 0.43 * score));
+        rows = 1e-3 * N * L * ((hot ? 0.088 : 0.137) * K + 0.09 * score);
+    } else if (token == TokenKernel::flow) {
+        const double whole = !flow_split_build(m.N, m.R, m.R2, m.L, call == ScanCall::score ? kModeScore : kModeRun);
+        alone = 5.1 * L + T * (0.52 + 0.62 * whole + 0.0086 * L * K + 0.52 * score);
+        rows = 1e-3 * N * L * ((hot ? 0.12 : 0.095) * K + 0.35 + 0.55 * whole + 0.5 * score);
+        alone *= alone, rows *= rows;      // (few calls between the two: nearer their maximum than the others)
+    } else if (token == TokenKernel::pipe) {
+        alone = L * (1.6 + 0.24 * P) + T * (0.8 + 0.31 * P + 0.019 * L * K + 1.2 * score);
+        rows = 3.3 + 1e-3 * N * L * ((hot ? 0.034 : 0.053) * K + 0.134 * P + 0.23 * score);
     } else {
-        scan += 11 * L + 1e-3 * N * (L - 1) * (0.25 + 0.137 * K);
+        alone = L * (2.1 + T * (0.74 + 0.0069 * K + 0.27 * P + 0.27 * score));
+        rows = 1e-3 * N * L * ((hot ? 0.052 : 0.1) * K + 0.18 * score);
     }
-    // token by token: a stream's token after token while the streams do not fill the chip, else its rows
-    const double token = m.K ? std::max(T * (10 + 0.45 * K), 1e-3 * N * L * 0.25 * K)
-                             : std::max(T * (0.5 + 0.055 * K) + (T < 32 ? 35 : 4.7 * L), 1e-3 * N * L * (0.11 + 0.124 * K));
-    return scan < token;
+    double by_token = std::hypot(alone, rows);
+    if (!m.K && token == TokenKernel::flow) by_token = std::sqrt(by_token);
+    // layer by layer: the launches, the recurrence's steps (whole runs of 16 tokens), its loads past each stream's end, the
+    // rows (past 4 MB of A16 an XCD's blocks outgrow its L2), the logits or the NLL
+    const double steps = (T + 15) / 16 * 16;
+    double scan = 3.3e-7 * B * L * n * n;
+    if (sort_pays(m, B * T)) {
+        const double E = std::max(m.E, m.V), miss = (double)m.E * n * 4 > 6e6 ? 2.5 : 1.0;
+        scan += L * (18.6 + 0.057 * steps + 0.0022 * E) + 1e-3 * N * ((L - 1) * 0.037 * K + 2.1e-3 * L * n * miss);
+        scan += out * (10.6 + N * (7e-5 + 1.4e-6 * m.V)) + score * (13 + 0.06 * T + 1.7e-4 * N);
+    } else {
+        scan += L * (8.5 + steps * (0.046 + 0.00016 * n)) + 1e-3 * N * (L - 1) * 0.145 * K;
+        scan += out * (9 + 2.1e-6 * N * m.V) + score * (5.5 + 0.054 * T + 2.4e-4 * N);
+    }
+    return scan < by_token;
 }
 
 int64_t scan_scratch_bytes(const YggDevModel &m, int64_t B, int64_t T, bool score, bool sort, int64_t cap) {

@@ -230,10 +230,11 @@ class Yggdrasil:
         g.replay()
         return logits.clone(), h.clone()
 
-    def _scratch(self, B: int, T: int, score: bool):
-        """(device scratch, its bytes) of a call that runs layer by layer over its known tokens (ygg_scratch), or
-        (None, 0) where it runs token by token: that is what the call takes, or there is no memory for the scratch."""
-        need = _lib.lib().ygg_scratch(self._h, B, T, int(score)) if T > 1 else 0
+    def _scratch(self, B: int, T: int, call: int):
+        """(device scratch, its bytes) of a call (0: run, 1: score, 2: run without logits) that goes layer by layer over
+        its known tokens (ygg_scratch), or (None, 0) where it goes token by token: that is what the call takes, or there
+        is no memory for the scratch."""
+        need = _lib.lib().ygg_scratch(self._h, B, T, call) if T > 1 else 0
         if not need:
             return None, 0
         try:
@@ -273,7 +274,7 @@ class Yggdrasil:
         else:
             dg = None
         scratch, need = (None, 0) if sv is not None or dg is not None or _entry != "ygg_run" else \
-            self._scratch(B, T, False)
+            self._scratch(B, T, 0 if logits else 2)
         if scratch is not None:
             check(_lib.lib().ygg_run_scratch(self._h, _ptr(x), B, T, _ptr(st), _ptr(lg), _ptr(lv), _ptr(scratch), need,
                                              _stream()))
@@ -328,7 +329,7 @@ class Yggdrasil:
                     xd, yd = xd[:, :-1].contiguous(), xd[:, 1:].contiguous()
                 else:
                     yd = self._tokens(targets[i:i + batch])
-                scratch, need = self._scratch(B, T, True)
+                scratch, need = self._scratch(B, T, 1)
                 if scratch is not None:
                     check(_lib.lib().ygg_score_scratch(self._h, _ptr(xd), _ptr(yd), B, T, _ptr(st), _ptr(nll),
                                                        _ptr(scratch), need, _stream()))
