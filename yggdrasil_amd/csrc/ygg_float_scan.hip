@@ -691,10 +691,11 @@ template <typename T> Plan plan_of(const FloatDevModel<T> &m, int64_t B) {
 
 // Calls of fewer than 4 tokens stay on the step kernel, and so do transition blocks other than 16. A model without a
 // step build of its own comes here from 4 tokens, where this form is far ahead of the general kernel: 4 tokens of 1 / 16 /
-// 256 / 1024 streams took (us, general kernel / this form), at depth 10 and 5 layers, n = 64, R = 12, R2 = 16 in f32 409/75
-// 417/85 412/97 1635/129; n = 256, R = R2 = 32 in f32 463/110 471/135 479/189 1905/354, in f64 506/135 513/166 525/327
-// 2078/491; n = 256, R = R2 = 64, 8 layers of depth 6, f64 852/266 865/343 887/507 3508/731; n = 16, 2 layers of depth 3, f32 105/24
-// 108/27 107/29 420/31; a token layer alone, n = 64, f64 55/15 55/19 57/19 218/24. (Fewer tokens were not compared.)
+// 256 / 1024 streams took (us, general kernel / this form), at depth 10 and 5 layers, n = 64, R = 12, R2 = 16 in f32 399/75
+// 411/82 399/95 1585/126; n = 256, R = R2 = 32 in f32 436/109 448/134 451/189 1799/345, in f64 492/133 499/165 503/324
+// 1995/490; n = 256, R = R2 = 64, 8 layers of depth 6, f64 817/265 830/343 850/505 3360/727; n = 16, 2 layers of depth 3,
+// f32 104/24 108/28 106/27 416/32; a token layer alone, n = 64, f64 55/16 56/18 56/18 221/24. (Fewer tokens were not
+// compared.)
 // With a step build (float_steps) the cheaper is estimated: a step's tokens, by rounds of the streams that fit the chip,
 // against this form's launches, the records its rows read (1.2 TB/s) and the sort. Measured at 4 and 8 tokens: small,
 // 1 stream 54/75 104/77, 256 58/96 112/105, 1024 71/150 139/169; medium 57/90 109/91, 76/125 146/146, 152/190 295/248;
